@@ -21,81 +21,22 @@
  * per workgroup in LDS; each chunk's scales in an LDS table; waves walk chunks
  * blocks * waves apart with a register ring running across chunk boundaries.  n_embd off a
  * multiple of 16, or x, codes or scale off the vector walk's alignment, take the same walk
- * with every piece read by aligned dwords and funnel-shifted (UA). */
+ * with every piece read by aligned dwords and funnel-shifted (UA).  Nine and more activation
+ * rows take the wide walk (r3d_logits_wide.h). */
 #include <hip/hip_runtime.h>
-#include <hip/hip_fp16.h>
 
 #include <mutex>
-#include <stddef.h>
 #include <stdio.h>
 #include <string.h>
 
 #include "r3d_device.h"
 #include "r3d_dump.h"
-#include "r3d_gemm_any.h"
+#include "r3d_logits_wide.h"
 #include "r3d_plan.h"
 #include "rad_planes.h"
 #include "rad_plugin.h"
 
 namespace r3d {
-
-typedef __bf16 lg_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 lg_bf16x2 __attribute__((ext_vector_type(2)));
-
-/* Eight e4m3 codes (two dwords, byte 0 first) -> eight bf16, exact. */
-__device__ __forceinline__ lg_bf16x8 lg_codes8(int w0, int w1) {
-    const lg_bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)w0, 1.0f, false);
-    const lg_bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)w0, 1.0f, true);
-    const lg_bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)w1, 1.0f, false);
-    const lg_bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)w1, 1.0f, true);
-    return lg_bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
-/* One scale element (bf16, f16 or f32 by SDT 0/1/2) at byte `off` of the plane, widened
- * exactly; an offset past the plane reads 0. */
-template <int SDT>
-__device__ __forceinline__ float lg_scale(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-    if (SDT == 2) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0));
-    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)off, 0, 0);
-    if (SDT == 0) return __uint_as_float(v << 16);
-    return __half2float(__ushort_as_half((unsigned short)v));
-}
-
-/* One scale element at any alignment (the dword walk): widened exactly. */
-template <int SDT>
-__device__ __forceinline__ float lg_scale_any(const AnyBuf& b, uint32_t off) {
-    const uint32_t v = any_ld4(b, off);
-    if (SDT == 2) return __uint_as_float(v);
-    if (SDT == 0) return __uint_as_float(v << 16);
-    return __half2float(__ushort_as_half((unsigned short)(v & 0xFFFFu)));
-}
-
-/* The device copy of the header still describes the planes the host planned from.  Read
- * by aligned dwords (the blob may start at any byte). */
-__device__ __forceinline__ bool lg_header_ok(const LogitsGuard& g) {
-    const int ne = (g.ic > g.is ? g.ic : g.is) + 1;
-    const uint32_t eb = (uint32_t)sizeof(RadPlanesHeader), es = (uint32_t)sizeof(RadPlanesEntry);
-    const AnyBuf hb = any_buf(g.header, eb + es * ne);
-    auto u32 = [&](uint32_t o) { return any_ld4(hb, o); };
-    auto i64 = [&](uint32_t o) {
-        return (int64_t)((uint64_t)any_ld4(hb, o) | ((uint64_t)any_ld4(hb, o + 4) << 32));
-    };
-    if (u32(offsetof(RadPlanesHeader, magic)) != RAD_PLANES_MAGIC ||
-        u32(offsetof(RadPlanesHeader, n_planes)) != 2)
-        return false;
-    const uint32_t c = eb + es * g.ic, s = eb + es * g.is;
-    return u32(c + offsetof(RadPlanesEntry, dtype)) == RAD_F8E4M3 &&
-           i64(c + offsetof(RadPlanesEntry, offset)) == g.c_off &&
-           i64(c + offsetof(RadPlanesEntry, rows)) == g.c_rows &&
-           i64(c + offsetof(RadPlanesEntry, cols)) == g.c_cols &&
-           u32(s + offsetof(RadPlanesEntry, dtype)) == g.s_dtype &&
-           i64(s + offsetof(RadPlanesEntry, offset)) == g.s_off &&
-           i64(s + offsetof(RadPlanesEntry, rows)) == g.s_rows &&
-           i64(s + offsetof(RadPlanesEntry, row_bytes)) == g.s_row_bytes &&
-           i64(s + offsetof(RadPlanesEntry, block)) == g.s_br;
-}
-
-constexpr uint32_t kLgOob = 0x80000000u;     /* past every buffer's num_records: reads 0 */
 
 /* A chunk is 16 head rows (four groups of 4) over the whole of K, walked in 256-wide
  * windows.  v_mfma_f32_16x16x32_bf16 sees 16 "rows" in source A; here A row i is (head row
@@ -551,6 +492,35 @@ static hipError_t launch_logits_dx(const LogitsPlan& P, hipStream_t s) {
                       : launch_logits_t<D, XG, 2, UA>(P, s);
 }
 
+/* The wide walk: P.wide groups of 16 activation rows a pass, P.wtw tiles a wave. */
+template <int NTG, int TW, int SDT>
+static hipError_t launch_wide_t(const LogitsPlan& P, hipStream_t stream) {
+    const int esz = SDT == 2 ? 4 : 2;
+    const int64_t s_bytes = P.guard.s_rows * P.s_pitch * esz;
+    const LogitsGeom g = logits_wide_geom(P, cu_count());
+    hipLaunchKernelGGL((logits_wide_kernel<NTG, TW, SDT>),
+                       dim3((unsigned)g.blocks, (unsigned)g.passes), dim3(512), (size_t)P.lds,
+                       stream, P.X, P.x_pitch, P.codes, P.scale, P.s_pitch, s_bytes, P.br, P.Y,
+                       P.y_pitch, (int)P.N, (int)P.K, (int)P.M, P.nwin, P.guard);
+    return hipGetLastError();
+}
+
+template <int NTG, int TW>
+static hipError_t launch_wide_s(const LogitsPlan& P, hipStream_t s) {
+    return P.sdt == 0 ? launch_wide_t<NTG, TW, 0>(P, s)
+         : P.sdt == 1 ? launch_wide_t<NTG, TW, 1>(P, s) : launch_wide_t<NTG, TW, 2>(P, s);
+}
+
+template <int TW>
+static hipError_t launch_wide_n(const LogitsPlan& P, hipStream_t s) {
+    return P.wide == 1 ? launch_wide_s<1, TW>(P, s) : P.wide == 2 ? launch_wide_s<2, TW>(P, s)
+         : P.wide == 3 ? launch_wide_s<3, TW>(P, s) : launch_wide_s<4, TW>(P, s);
+}
+
+static hipError_t launch_logits_wide(const LogitsPlan& P, hipStream_t s) {
+    return P.wtw == 2 ? launch_wide_n<2>(P, s) : launch_wide_n<1>(P, s);
+}
+
 template <bool UA>
 static hipError_t launch_logits_u(const LogitsPlan& P, hipStream_t stream) {
     /* 5..8 activation rows a pass: two groups of 4, one window in flight (the plan's rule) */
@@ -571,7 +541,8 @@ static int logits_entry(const RadArgs* a, RadStream s) {
     if (rc) return rc;
     rc = plan_logits_e4m3(a, &hc, &P, false);
     if (rc) return rc;
-    const hipError_t e = P.ua ? launch_logits_u<true>(P, stream) : launch_logits_u<false>(P, stream);
+    const hipError_t e = P.wide ? launch_logits_wide(P, stream)
+                       : P.ua ? launch_logits_u<true>(P, stream) : launch_logits_u<false>(P, stream);
     if (e != hipSuccess) {
         fprintf(stderr, "libr3d_gfx950: logits_e4m3 launch FAILED (%s)\n", hipGetErrorName(e));
         return RAD_E_DEVICE;

@@ -1085,6 +1085,16 @@ int plan_logits_e4m3(const RadArgs* a, const RadPlanesHead* hh, LogitsPlan* P, b
     P->s_pitch = es->row_bytes / ssz;
     P->y_pitch = y_pitch;
     P->lds = (int)(sh.mt * sh.xrow + sh.stab);
+    /* past 8 rows the 4-row walk streams the head again for every 8; the wide walk serves 64
+     * a pass.  Not at 8: there one pass of the 4-row walk costs the same (262144 x 5376: 236
+     * against 232 us; 151936 x 4096: 122 against 124).  Heads under 128 blocks of 128 rows
+     * leave too few workgroups in flight for its window-by-window barrier.  One pass's x
+     * offsets are 32-bit. */
+    if (!P->ua && M > 8 && N >= 128 * 128 && 2 * 64 * x_pitch < 0x7FFFFFFFLL) {
+        P->wide = (int)(M >= 64 ? 4 : (M + 15) / 16);
+        P->wtw = logits_wide_tiles(N, P->wide, cu_count());
+        P->lds = logits_wide_lds(P->wide);
+    }
     LogitsGuard& g = P->guard;
     g.header = (const uint8_t*)W->data;
     g.ic = (int32_t)(ec - rad_planes_entries(h));
@@ -1102,6 +1112,28 @@ LogitsGeom logits_geom(const LogitsPlan& P, int cus, int per_cu) {
     if (blocks > (int64_t)cus * per_cu) blocks = (int64_t)cus * per_cu;
     g.blocks = (int)blocks;
     g.passes = (P.M + P.mt - 1) / P.mt;
+    return g;
+}
+
+/* Tiles a wave of the wide walk.  Two halve the restaging of the activation rows; one deals
+ * the head over the 2 x cus workgroups in blocks half the size.  A round of one-tile blocks
+ * costs a half of a two-tile round and f more (262144 x 5376, 4 rounds against 2 x 2: 1.07 at
+ * 16 activation rows, 1.13 at 32, 1.23 at 64), so one tile runs where its rounds cost less:
+ * 151936 x 4096 (3 rounds against 2 x 2) M = 16 132 against 146 us, M = 32 144 against 156,
+ * but M = 64 183 against 175; 32000 x 4096 (1 against 2 x 1) 31 against 42 and, at 64, 41
+ * against 52. */
+int logits_wide_tiles(int64_t N, int ntg, int cus) {
+    const int64_t wgs = 2 * (int64_t)(cus > 0 ? cus : 256);
+    const int64_t r1 = ((N + 127) / 128 + wgs - 1) / wgs, r2 = ((N + 255) / 256 + wgs - 1) / wgs;
+    return r1 * (ntg <= 2 ? 115 : 140) < 2 * r2 * 100 ? 1 : 2;
+}
+
+LogitsGeom logits_wide_geom(const LogitsPlan& P, int cus) {
+    LogitsGeom g{};
+    g.chunks = (P.N + 128 * P.wtw - 1) / (128 * P.wtw);
+    const int64_t wgs = 2 * (int64_t)(cus > 0 ? cus : 256);
+    g.blocks = (int)(g.chunks < wgs ? g.chunks : wgs);
+    g.passes = (P.M + 63) / 64;
     return g;
 }
 
@@ -1220,13 +1252,14 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
         }
         if (!rc) rc = plan_logits_e4m3(a, &hc, &L, false);
         if (rc) { snprintf(buf, (size_t)len, "refused rc=%d (plan)", rc); return rc; }
-        const LogitsGeom g = logits_geom(L, 256, 1);
+        const LogitsGeom g = L.wide ? logits_wide_geom(L, 256) : logits_geom(L, 256, 1);
         snprintf(buf, (size_t)len,
                  "arm=logits M=%lld N=%lld K=%lld mt=%d passes=%lld depth=%d wg_waves=%d "
                  "chunks=%lld blocks=%d br=%d sdt=%d nwin=%d lds=%d walk=%s",
-                 (long long)L.M, (long long)L.N, (long long)L.K, L.mt, (long long)g.passes,
-                 L.depth, L.waves, (long long)g.chunks, g.blocks, L.br, L.sdt, L.nwin, L.lds,
-                 L.ua ? "dword" : "vector");
+                 (long long)L.M, (long long)L.N, (long long)L.K, L.wide ? 16 * L.wide : L.mt,
+                 (long long)g.passes, L.wide ? 1 : L.depth, L.wide ? 8 : L.waves,
+                 (long long)g.chunks, g.blocks, L.br, L.sdt, L.nwin, L.lds,
+                 L.wide == 0 ? (L.ua ? "dword" : "vector") : L.wtw == 2 ? "wide2" : "wide1");
         return RAD_OK;
     }
     if (strstr(row, "rmsnorm_quant_fp8") != nullptr) {

@@ -345,6 +345,8 @@ struct LogitsPlan {
     int lds;                 /* dynamic LDS bytes per workgroup: x rows, then scale tables */
     int ua;                  /* n_embd off a multiple of 16, or x / codes / scale off the fast
                                 walk's alignment: every piece read by dwords, funnel-shifted */
+    int wide, wtw;           /* the wide walk's 16-row activation groups (1..4; 0: the 4-row
+                                walk) and 16-row head tiles a wave (1, 2) */
     LogitsGuard guard;
 };
 /* `h` null: the gates that need no header (args_only); else a host copy of the blob's
@@ -372,6 +374,12 @@ struct LogitsGeom {
     int64_t passes;
 };
 LogitsGeom logits_geom(const LogitsPlan& P, int cus, int per_cu);
+/* The wide walk (r3d_logits_wide.h): its LDS at ntg activation groups (two windows of x, then
+ * 8 waves' scale tables), its tiles a wave, and its grid (two workgroups a compute unit,
+ * chunks counting blocks of 128 wtw head rows; passes of 64 activation rows). */
+constexpr int logits_wide_lds(int ntg) { return 2 * 8192 * ntg + 8 * 2 * 256; }
+int logits_wide_tiles(int64_t N, int ntg, int cus);
+LogitsGeom logits_wide_geom(const LogitsPlan& P, int cus);
 
 /* The current device: gfx950 or not (answered once per device), and its compute units. */
 bool chip_ok();

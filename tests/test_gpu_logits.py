@@ -125,6 +125,28 @@ def test_logits_parity(gpu, M, N, K, sdt, br, xp, yp):
     check(Y, x, codes, sbits, sdt, br, "logits_M%d_N%d_K%d_%s_br%d" % (M, N, K, sdt, br))
 
 
+WIDE = [  # M, N, K, sdt, br, x_pitch, y_pitch: the wide walk (9 rows up, 16384 head rows up)
+    (9, 16384, 256, "bf16", 1, None, None),      # one window, the smallest head
+    (16, 16387, 144, "f16", 1, None, None),      # ragged N and a 16-wide last scale block
+    (17, 16500, 400, "bf16", 128, 408, 16501),   # two groups, odd logits pitch: scalar stores
+    (33, 16640, 272, "f32", 1, None, 16644),     # three groups
+    (64, 16385, 640, "bf16", 1, None, None),     # four groups, a block with one live row
+    (70, 16401, 208, "f32", 128, None, None),    # a second pass of six rows
+    (12, 65600, 512, "bf16", 1, None, None),     # one-tile blocks, more blocks than workgroups
+    (40, 131072, 256, "bf16", 1, None, None),    # two-tile blocks, one each
+]
+
+
+@pytest.mark.parametrize("M,N,K,sdt,br,xp,yp", WIDE)
+def test_logits_wide_parity(gpu, M, N, K, sdt, br, xp, yp):
+    print("logits wide parity M=%d N=%d K=%d %s br=%d" % (M, N, K, sdt, br), flush=True)
+    codes, sbits = LU.head(N, K, M * 7 + N, sdt, br)
+    x = synth.bf16_bits(np.random.default_rng(M + K).standard_normal((M, K)).astype(np.float32))
+    rc, Y, ok = run(x, codes, sbits, sdt, br, gpu, xp, yp)
+    assert rc == R.RAD_OK and ok
+    check(Y, x, codes, sbits, sdt, br, "logits_wide_M%d_N%d_K%d_%s_br%d" % (M, N, K, sdt, br))
+
+
 @pytest.mark.parametrize("sdt,br,pad,shift", [("bf16", 1, 3, 0), ("f16", 1, 0, 2),
                                               ("f32", 1, 1, 4), ("bf16", 128, 5, 6)])
 def test_scale_plane_layouts(gpu, sdt, br, pad, shift):

@@ -122,6 +122,24 @@ def test_plan_geometry():
     assert _desc(ops)[0] == R.RAD_OK                  # constraint is the resolver's, not a gate
 
 
+def test_plan_wide_walk():
+    """Past 8 activation rows a head of 16384 rows up takes the wide walk: 64 rows a pass, two
+    tiles a wave unless one-tile blocks' rounds over the 512 workgroups cost less.  8 rows, a
+    small head, or operands off the vector walk's alignment keep the 4-row walk."""
+    for M, N, walk, mt, passes in [(9, 262144, "wide2", 16, 1), (16, 151936, "wide1", 16, 1),
+                                   (64, 151936, "wide2", 64, 1), (33, 32000, "wide1", 48, 1),
+                                   (65, 16384, "wide1", 64, 2), (8, 262144, "vector", 8, 1),
+                                   (16, 16383, "vector", 8, 2)]:
+        ops, keep = _ops(M=M, N=N, K=256)
+        rc, g = _desc(ops)
+        assert rc == R.RAD_OK and g["walk"] == walk, (M, N, g)
+        assert (g["mt"], g["passes"]) == (str(mt), str(passes)), (M, N, g)
+        if walk.startswith("wide"):
+            assert g["lds"] == str(1024 * mt + 4096), g
+    ops, keep = _ops(M=16, N=16384, K=260)
+    assert _desc(ops)[1]["walk"] == "dword"
+
+
 def _hdr(N=1000, K=5376, sdt="bf16", br=1, **fields):
     h = LU.header(N, K, sdt, br)
     for key, v in fields.items():
