@@ -24,6 +24,7 @@
 #include "r3d_gemv_wide.h"
 #include "r3d_plan.h"
 #include "r3d_prefill.h"
+#include "r3d_prefill_f8.h"
 #include "rad_plugin.h"
 
 namespace r3d {
@@ -232,6 +233,34 @@ static hipError_t splitk_reduce(const GemmPlan& P, int kc, const float* part, hi
     return hipGetLastError();
 }
 
+/* The fp8a8 wide tile (prefill_f8_kernel) of 256 x 32 wmw over kc chunks of cst groups: into
+ * bf16 Y (kc = 1), or f32 partial planes at part. */
+static hipError_t launch_f8_wide(const GemmPlan& P, int wmw, int kc, int cst, float* part,
+                                 hipStream_t stream) {
+    const int64_t gn = (P.N + 255) / 256, gm = (P.M + 32 * wmw - 1) / (32 * wmw);
+    /* 32-bit lane offsets over 256 rows of every operand */
+    const int64_t lim = (int64_t)1 << 31;
+    if (256 * P.a_pitch >= lim || 256 * P.b_pitch >= lim || 512 * P.bs_pitch >= lim ||
+        1024 * P.as_pitch >= lim || gn * gm * kc > 0x7FFFFFFF || kc < 1 || cst < 1 || P.M < 1)
+        return hipErrorInvalidValue;
+    const F8Args a{P.A, P.AS, P.B, (const uint16_t*)P.BS, P.Y, (int)P.M, (int)P.N, P.a_pitch,
+                   P.as_pitch, P.b_pitch, P.bs_pitch, P.y_pitch, kc > 1 ? part : nullptr};
+    const dim3 grid((unsigned)(gn * gm * kc)), block(512);
+#define R3D_F8W(W_, R_)                                                                     \
+    hipLaunchKernelGGL((prefill_f8_kernel<W_, R_>), grid, block,                             \
+                       (size_t)PrefillF8Layout<W_>::LDS_ALL, stream, a, (int)(P.K / 128),    \
+                       (int)gm, (int)(gn * gm), kc, cst)
+    if (wmw == 8) {
+        if (P.rblk == 128) R3D_F8W(8, 128); else R3D_F8W(8, 1);
+    } else if (wmw == 4) {
+        if (P.rblk == 128) R3D_F8W(4, 128); else R3D_F8W(4, 1);
+    } else {
+        return hipErrorInvalidValue;
+    }
+#undef R3D_F8W
+    return hipGetLastError();
+}
+
 /* The skinny-band GEMV's K split, then the reduce; RAD_OK, or RAD_E_DEVICE (reported as
  * `what`) when a launch fails, for the caller's unsplit arms to recompute every element of
  * Y.  decode: the decode rows' split (named so in the R3D_DEBUG_GEMM line). */
@@ -362,7 +391,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
                          ? splitk_plan(P.enc, P.M, P.N, P.K, cu_count(), &kc, &cst, &gs, &gw)
                          : 0;
     const bool split = kind != 0 && part_bytes >= (int64_t)kc * P.M * P.N * 4 &&
-                       (kind == 1 || (gs.grid_m == 1 && gs.tiles * kc <= 0x7FFFFFFF));
+                       (kind != 2 || (gs.grid_m == 1 && gs.tiles * kc <= 0x7FFFFFFF));
     /* the skinny band on a narrow N: 16-row passes of the decode GEMVs (each output row is
      * the same arithmetic either way) */
     if (const int passes = split || P.ua ? 0 : skinny_passes(P.enc, P.M, P.N, cu_count())) {
@@ -446,7 +475,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
                 case 8: R3D_PF(PF_MX8, 8, 4); break;
                 case 7: R3D_PF(PF_MX8, 7, 4); break;
                 case 6: R3D_PF(PF_MX8, 6, 4); break;
-                default: R3D_PF(PF_MX8, 4, 4); break;
+                default: if (g.wmf == 2) { R3D_PF(PF_MX8, 4, 2); } else { R3D_PF(PF_MX8, 4, 4); } break;
             }
         } else if (mode == PF_F8 && Q.rblk == 128) {
             /* the 128 x 128 block grid: one weight scale a tile and K group, folded into
@@ -494,7 +523,9 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
         hipError_t e = hipSuccess;
         if (forced_fail("splitk")) {
             launch_failed("split-K prefill", hipSuccess);
-        } else if ((e = tiles_launch(gs, kc, cst, reinterpret_cast<float*>(part), P)) !=
+        } else if ((e = kind == 3 ? launch_f8_wide(P, gs.wmf, kc, cst,
+                                                   reinterpret_cast<float*>(part), stream)
+                                  : tiles_launch(gs, kc, cst, reinterpret_cast<float*>(part), P)) !=
                    hipSuccess) {
             launch_failed("split-K prefill", e);
         } else if ((e = splitk_reduce(P, kc, reinterpret_cast<const float*>(part), stream)) !=
@@ -506,6 +537,16 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
             return RAD_OK;
         }
         /* a failed split: the whole K walk below recomputes every element of Y */
+    }
+    /* e4m3 weights past 128 tokens: the wide tile where its rounds cost less (a failed launch
+     * leaves every element of Y to the tiles below) */
+    if (const int w = mode == PF_F8 ? prefill_f8_wide(P.M, P.N, P.K, P.rblk, cu_count()) : 0) {
+        const hipError_t e = launch_f8_wide(P, w, 1, (int)(P.K / 128), nullptr, stream);
+        if (e == hipSuccess) {
+            debug_once("fp8a8 prefill, wide tile", 180 + w);
+            return RAD_OK;
+        }
+        launch_failed("wide-tile prefill", e);
     }
     /* e4m3 weights on the four-wave tile: whole rounds of it over the first n1 weight rows,
      * the rest on the 128 x 128 tile (prefill_f8_split_n) */

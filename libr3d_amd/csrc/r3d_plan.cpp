@@ -556,6 +556,90 @@ int64_t prefill_f8_split_n(int64_t M, int64_t N, int ncu) {
     return 171 * r1 + 100 * r2 < 171 * rall ? 128 * n1t : 0;
 }
 
+/* What an fp8a8 prefill takes, in ns, from least squares over 150 shapes (M 144..2048, N
+ * 737..21504, K 1024..21504; 9 % mean error): a round of 256 workgroups of each tile, and a
+ * split's planes, written and read back, with the reduce launch. */
+static int64_t f8_rounds(int64_t tiles, int ncu) { return (tiles + ncu - 1) / ncu; }
+struct F8Cost {
+    int64_t a, b;            /* a round: a + b * steps */
+};
+static const F8Cost kF8Base = {4600, 575}, kF8Wide8 = {8200, 1420}, kF8Wide4 = {5400, 950};
+/* the per-row grid with scales that do vary along a row, the wide tile's slower walk */
+static const F8Cost kF8BaseRow = {4600, 760}, kF8Wide8Row = {8200, 2500}, kF8Wide4Row = {5400, 1450};
+
+/* prefill_geom's tiles: 128 x 128 rounds, or 128 x 256 ones with or without a remainder */
+static int64_t f8_base_ns(const F8Cost& c, int64_t M, int64_t N, int64_t steps, int ncu) {
+    const int64_t rn = (N + 127) / 128;
+    const int64_t r1 = 100 * f8_rounds(rn * ((M + 127) / 128), ncu);
+    int64_t r4 = 171 * f8_rounds(rn * ((M + 255) / 256), ncu);
+    if (const int64_t n1 = prefill_f8_split_n(M, N, ncu))
+        r4 = 171 * f8_rounds((n1 / 128) * ((M + 255) / 256), ncu) +
+             100 * f8_rounds((N - n1 + 127) / 128 * ((M + 127) / 128), ncu);
+    return (r4 < r1 ? r4 : r1) * (c.a + c.b * steps) / 100;
+}
+static int64_t f8_wide_ns(const F8Cost& c, int wmw, int64_t M, int64_t N, int64_t steps, int64_t kc,
+                          int ncu) {
+    const int64_t tiles = ((N + 255) / 256) * ((M + 32 * wmw - 1) / (32 * wmw));
+    return f8_rounds(tiles * kc, ncu) * (c.a + c.b * steps);
+}
+
+int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu) {
+    if (M <= 128 || f8_tile_lever()) return 0;
+    if (ncu <= 0) ncu = 256;
+    /* On the per-row grid the host cannot see whether the scales vary, so the wide tile runs
+     * where even its slower walk gains: M = 512, N = 21504, K = 5376 stays on the base tiles
+     * (109 us; the wide tile 93 with one scale a row, 128 with scales that vary). */
+    const bool row = rblk == 1;
+    const int64_t steps = K / 128;
+    const int64_t base = f8_base_ns(row ? kF8BaseRow : kF8Base, M, N, steps, ncu);
+    const int64_t c8 = f8_wide_ns(row ? kF8Wide8Row : kF8Wide8, 8, M, N, steps, 1, ncu);
+    const int64_t c4 = f8_wide_ns(row ? kF8Wide4Row : kF8Wide4, 4, M, N, steps, 1, ncu);
+    return c8 <= c4 ? (c8 < base ? 8 : 0) : c4 < base ? 4 : 0;
+}
+
+int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g) {
+    if (M < kPrefillSplitM || f8_tile_lever()) return 0;
+    if (ncu <= 0) ncu = 256;
+    const int64_t steps = K / 128;
+    int64_t best = f8_base_ns(kF8Base, M, N, steps, ncu), kbest = 0;
+    for (int w = 4; w <= 8; w += 4) {
+        const int64_t c = f8_wide_ns(w == 8 ? kF8Wide8 : kF8Wide4, w, M, N, steps, 1, ncu);
+        if (c < best) best = c;
+    }
+    /* a split that is close gives way to the single launch (within the model's error they lost
+     * up to 22 %: M = 2048, N = 737, K = 5376, 32 against 39 us) */
+    best = best * 88 / 100;
+    int wbest = 0;
+    for (int w = 4; w <= 8; w += 4) {
+        const int64_t tiles = ((N + 255) / 256) * ((M + 32 * w - 1) / (32 * w));
+        for (int64_t kc = 2; kc <= 32 && steps / kc >= 3 && tiles * kc <= 2 * ncu; ++kc) {
+            const int64_t cs = (steps + kc - 1) / kc, kk = (steps + cs - 1) / cs;
+            const int64_t bytes = kk * M * N * 4;
+            if (kk != kc || bytes > kPrefillSplitMaxBytes) continue;
+            const int64_t c = f8_wide_ns(w == 8 ? kF8Wide8 : kF8Wide4, w, M, N, cs, kk, ncu) +
+                              5400 + bytes * 28 / 100000;
+            if (c < best) { best = c; kbest = kk; wbest = w; }
+        }
+    }
+    if (!kbest) return 0;
+    if (cst) *cst = (int)((steps + kbest - 1) / kbest);
+    if (g) {
+        *g = PrefillGeom{};
+        g->wnf = 4;
+        g->wmf = wbest;
+        g->nst = 2;
+        g->wv = 8;
+        g->bn = 256;
+        g->bm = 32 * wbest;
+        g->grid_n = (N + 255) / 256;
+        g->grid_m = (M + g->bm - 1) / g->bm;
+        g->tiles = g->grid_n * g->grid_m;
+        g->steps = (int)steps;
+        g->lds = wbest == 8 ? PrefillF8Layout<8>::LDS_ALL : PrefillF8Layout<4>::LDS_ALL;
+    }
+    return (int)kbest;
+}
+
 int skinny_passes(int enc, int64_t M, int64_t N, int ncu) {
     if ((enc != ENC_MXFP4A8 && enc != ENC_FP8A8) || M < 17 || M > 64) return 0;
     static const int lever = [] {
@@ -637,6 +721,14 @@ static bool wide_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t kc0, Wid
 
 int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int* cst,
                 PrefillGeom* g, WideGeom* w) {
+    if (enc == ENC_FP8A8 && M > 128 && N > 0 && K >= 128) {
+        int c = 0;
+        const int k = prefill_f8_splitk(M, N, K, ncu, &c, g);
+        if (!k) return 0;
+        if (kc) *kc = k;
+        if (cst) *cst = c;
+        return 3;
+    }
     if ((enc != ENC_MXFP4A8 && enc != ENC_FP8A8) || M < 1 || M > 128 || N < 1 || K < 128)
         return 0;
     static const bool tile_only = [] {
@@ -683,8 +775,7 @@ int64_t tile_scratch_bytes(const RadArgs* a, int enc, int ncu) {
     long long N = 0, K = 0, M = 0;
     if (!rad_args_geti(a, "N", &N) || !rad_args_geti(a, "K", &K)) return 0;
     if (N <= 0 || K <= 0 || N > (1LL << 34) || K > (1LL << 27)) return 0;
-    /* the launch's own M (numel(y) / N) when y is there, else the M parameter, else the
-     * largest M the split takes */
+    /* the launch's own M (numel(y) / N) when y is there, else the M parameter, else 128 */
     const RadTensor* Y = rad_arg_in(a, 4);
     const long long yn = Y ? rad_tensor_numel(Y) : 0;
     if (yn > 0 && yn % N == 0)
@@ -1379,11 +1470,11 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
             wide_line(w, kc, "splitk");
         else
             snprintf(buf, (size_t)len,
-                     "arm=splitk kernel=tile enc=%s M=%lld N=%lld K=%lld bn=%d bm=%d tiles=%lld "
+                     "arm=splitk kernel=%s enc=%s M=%lld N=%lld K=%lld bn=%d bm=%d tiles=%lld "
                      "kc=%d cst=%d steps=%d lds=%d partials=%lld (f32 partial planes in scratch, "
                      "summed in chunk order)",
-                     ename, (long long)P.M, (long long)P.N, (long long)P.K, g.bn, g.bm,
-                     (long long)g.tiles, kc, cst, g.steps, g.lds, (long long)kc * P.M * P.N * 4);
+                     kind == 3 ? "f8wide" : "tile", ename, (long long)P.M, (long long)P.N,
+                     (long long)P.K, g.bn, g.bm, (long long)g.tiles, kc, cst, g.steps, g.lds, (long long)kc * P.M * P.N * 4);
     } else if (const int passes = skinny_passes(P.enc, P.M, P.N, 256)) {
         snprintf(buf, (size_t)len,
                  "arm=skinny enc=%s M=%lld N=%lld K=%lld passes=%d (16-row decode GEMV passes)",
@@ -1392,14 +1483,17 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
         const int mode = a16 ? PF_MX8 : mx ? PF_A8 : PF_F8;
         PrefillGeom g{};
         prefill_geom(P.M, P.N, P.K, mode, 256, &g);
+        const int fw = mode == PF_F8 ? prefill_f8_wide(P.M, P.N, P.K, P.rblk, 256) : 0;
         snprintf(buf, (size_t)len,
                  "arm=prefill enc=%s M=%lld N=%lld K=%lld bn=%d bm=%d waves=%d grid=%lldx%lld "
-                 "tiles=%lld nst=%d lds=%d steps=%d rblk=%d nsplit=%lld quant=%s",
+                 "tiles=%lld nst=%d lds=%d steps=%d rblk=%d nsplit=%lld quant=%s%s",
                  ename, (long long)P.M, (long long)P.N, (long long)P.K, g.bn, g.bm, g.wv,
                  (long long)g.grid_n, (long long)g.grid_m, (long long)g.tiles, g.nst, g.lds,
                  g.steps, P.rblk,
                  (long long)(mode == PF_F8 && g.wv == 4 ? prefill_f8_split_n(P.M, P.N, 256) : 0),
-                 !a16 ? "none" : (P.ua & UA_QUANT) ? "elementwise" : "vector");
+                 !a16 ? "none" : (P.ua & UA_QUANT) ? "elementwise" : "vector",
+                 /* the tile that takes the launch, ahead of the ones above */
+                 fw == 8 ? " wide=256x256" : fw == 4 ? " wide=256x128" : "");
     }
     return RAD_OK;
 }

@@ -201,6 +201,16 @@ int skinny_passes(int enc, int64_t M, int64_t N, int ncu);
  * 1.71 rounds of the other).  Returns n1 (a multiple of 128), or 0 for one launch over N. */
 int64_t prefill_f8_split_n(int64_t M, int64_t N, int ncu);
 
+/* The fp8a8 wide tile (r3d_prefill_f8.h) for an unsplit launch: its token fragments a wave
+ * (8: 256 x 256, 4: 256 x 128) past 128 tokens where its rounds cost less than the tiles of
+ * prefill_geom, else 0 (R3D_GFX950_F8_TILE keeps those).  rblk: the weight scale grid. */
+int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu);
+/* The same tile with K split over launch scratch, from kPrefillSplitM tokens: kc, or 0; *cst
+ * groups a chunk, *g the tile. */
+constexpr int64_t kPrefillSplitM = 144;
+constexpr int64_t kPrefillSplitMaxBytes = int64_t(256) << 20;
+int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g);
+
 /* The skinny-band GEMV (gemv_wide_kernel, r3d_gemv_wide.h): 8 waves of tw 16-row weight
  * tiles (256 rows a workgroup at tw = 2) x one K chunk of cg groups; depth d lines in each
  * wave's register ring (1: measured at least as fast as 2 and 4 on every config 2 shape at
@@ -223,8 +233,9 @@ constexpr int kWideMaxLds = 152 * 1024;
  * least kSplitMinSteps steps a chunk. */
 constexpr int kSplitMinSteps = 4;
 int tile_splitk(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g);
-/* The split's kernel: up to M = 64 the skinny-band GEMV (kind 1, *w), else the 128 x 128
- * prefill tile (kind 2, *g); 0 when no split applies.  *kc and *cst as tile_splitk's.
+/* The split's kernel: up to M = 64 the skinny-band GEMV (kind 1, *w), to 128 the 128 x 128
+ * prefill tile (kind 2, *g), past that the fp8a8 wide tile (kind 3, *g); 0 when no split
+ * applies.  *kc and *cst as tile_splitk's.
  * R3D_GFX950_SPLITK_KERNEL=tile keeps the prefill tile (64 tokens a tile) up to M = 64. */
 int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int* cst,
                 PrefillGeom* g, WideGeom* w);

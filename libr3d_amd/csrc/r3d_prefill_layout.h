@@ -44,6 +44,23 @@ constexpr int prefill_stage_bytes(int wnf, int wmw, int wh = 1, int wv = 8) {
     return wv * ((wh * 2 * wnf + wv - 1) / wv) * 1024 + 1024 + 8 * wv * wmw * 128 + 1024;
 }
 
+/* The fp8a8 wide tile (r3d_prefill_f8.h): 256 weight rows x 32 WMW tokens, a ring of two
+ * stages; the bf16 output tile, YP bytes a token, reuses it. */
+template <int WMW>
+struct PrefillF8Layout {
+    static constexpr int BN = 256, BM = 32 * WMW;
+    static constexpr int WLD = BN / 64, ALD = BM / 64, LOADS = WLD + ALD + 2;
+    static constexpr int W = 0;                   /* [BN/16][2 halves][1 KB] weights */
+    static constexpr int S = W + BN * 128;        /* [256] dwords: a weight row's bf16 scale */
+    static constexpr int A = S + 1024;            /* [BM/16][2 halves][1 KB] activations */
+    static constexpr int AS = A + BM * 128;       /* [256] dwords: a token's f32 scale */
+    static constexpr int STAGE = AS + 1024;
+    static constexpr int YP = 2 * BN + 32;        /* 32 mod 128: conflict-free 8-byte writes */
+    static constexpr int LDS = 2 * STAGE > BM * YP ? 2 * STAGE : BM * YP;
+    static constexpr int LDS_ALL = LDS + 64;      /* and eight waves' flags */
+    static_assert(LDS_ALL <= 160 * 1024, "ring exceeds the CU's LDS");
+};
+
 }  // namespace r3d
 
 #endif /* R3D_PREFILL_LAYOUT_H */

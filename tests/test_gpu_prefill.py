@@ -138,3 +138,66 @@ def test_mxfp4a16_short_scratch_refused(gpu):
     rc, Y, _, _, ok = run_a16(X, B, BS, M, N, K, gpu, scratch_bytes=M * K)
     assert rc == R.RAD_E_UNSUPPORTED and ok
     assert np.all(Y == _gu().Y_SENTINEL)                    # nothing launched
+
+
+F8_WIDE = [  # M, N, K, scratch: the fp8a8 wide tile, whole K and split
+    (1030, 8200, 128, None),      # 256 x 256: one step, six live tokens in the last tile, ragged N
+    (1030, 8448, 256, None),      # 256 x 256: two steps
+    (300, 21700, 384, None),      # 256 x 128: an odd step count, ragged M and N
+    (144, 300, 21504, "hook"),    # split: the least M, a ragged N past one tile
+    (500, 2050, 5376, "hook"),    # split, N off a multiple of 4
+    (513, 1000, 8192, "hook"),    # split, one live token in the last tile
+]
+
+
+@pytest.mark.parametrize("scales", ["block", "channel", "vary", "late"])
+@pytest.mark.parametrize("M,N,K,scratch", F8_WIDE)
+def test_fp8_wide_tile(gpu, M, N, K, scratch, scales):
+    """The wide tile at its edges, on both scale grids; on the per-row grid with one scale a row
+    (applied once after the walk), with scales that vary everywhere, and with one row's scale
+    that differs in its last group alone (that row's tile must take the per-group walk)."""
+    from tests.test_gpu_gemm import F8_TILE, _check, _f8_case
+    rblk = 128 if scales == "block" else 1
+    A, AS, B, BS = _f8_case(M, N, K, M + N + K, rblk)
+    if scales in ("channel", "late"):
+        BS = np.repeat(BS[:, :1], K // 128, axis=1).copy()
+    if scales == "late":
+        BS[N - 1, -1] += 0x80                              # twice as large
+    A, AS, B, BS = (np.ascontiguousarray(t) for t in (A, AS, B, BS))
+    if not _wide_route(M, N, K, rblk, scratch):
+        pytest.skip("the planner keeps the base tiles at this shape and grid")
+    _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk, scratch=scratch)
+
+
+def _wide_route(M, N, K, rblk, scratch):
+    rows = N if rblk == 1 else (N + 127) // 128
+    z = lambda *s, dt=torch.uint8: torch.zeros(s, dtype=dt)
+    ops = R.GemmOperands(z(M, K), z(M, K // 128, dt=torch.float32), z(N, K),
+                         z(rows, K // 128, dt=torch.int16), z(M, N, dt=torch.int16),
+                         dtype="fp8a8", N=N, K=K)
+    if scratch:
+        need = R.row_scratch_bytes("gemm_nt_q_fp8a8", ops)
+        if not need:
+            return False
+        ops.set_scratch(z(64), need)
+    d = R.describe("gemm_nt_q_fp8a8", ops)[1]
+    return "kernel=f8wide" in d if scratch else "wide=" in d
+
+
+@pytest.mark.parametrize("bad", [0x7F80, 0x7FC0])
+def test_fp8_wide_tile_non_finite_row_scale(gpu, bad):
+    """A row whose scale is Inf or NaN in every group is one scale a row, but its sum is not
+    sum(D * sa) * sb: it takes the per-group walk, NaN and Inf classes as the oracle's."""
+    from tests.test_gpu_gemm import F8_TILE, _f8_case
+    from tests import gpu_util as gu
+    M, N, K = 500, 2050, 5376
+    A, AS, B, BS = _f8_case(M, N, K, 5, 1)
+    BS = np.repeat(BS[:, :1], K // 128, axis=1).copy()
+    BS[700, :] = bad
+    rc, Y, ok = gu.run_row(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, scratch="hook")
+    assert rc == R.RAD_OK and ok
+    rows = slice(640, 768)                                 # the row's neighbours too
+    Yr, Yf, S = O.quant_dot_fp8a8(A, AS, B[rows], BS[rows], 1, nthreads=16)
+    S8 = O.group8_mag("fp8a8", A, AS, B[rows], BS[rows], 1, nthreads=16)
+    c = gu.compare(np.ascontiguousarray(Y[:, rows]), Yr, Yf, S, K, S8)
+    assert c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0 and c["max_viol"] <= 1.0, c
