@@ -498,7 +498,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
         } else if (g.wmf == 1) {
             R3D_PF(PF_A8, 8, 1);                        /* split K up to 64 tokens */
         } else if (g.wmf == 2) {
-            R3D_PF(PF_A8, 4, 2);                        /* up to 128 tokens */
+            R3D_PF(PF_A8, 4, 2);                        /* up to 128 tokens, or few tiles */
         } else {
             switch (g.wnf) {
                 case 8: R3D_PF(PF_A8, 8, 4); break;
@@ -532,7 +532,8 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
                    hipSuccess) {
             launch_failed("split-K reduce", e);
         } else {
-            debug_once(mode == PF_F8 ? "fp8a8 split-K prefill" : "mxfp4a8 split-K prefill",
+            debug_once(mode == PF_F8 ? "fp8a8 split-K prefill"
+                       : mode == PF_MX8 ? "mxfp4a16 split-K prefill" : "mxfp4a8 split-K prefill",
                        200 + 8 * mode + kind);
             return RAD_OK;
         }
@@ -581,6 +582,12 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
     return RAD_OK;
 }
 
+/* The bf16-in row: whatever the scratch holds past the quantised activations is the split's. */
+static int launch_mxfp4a16(const RadArgs* a, const GemmPlan& P, hipStream_t stream, int stage) {
+    const int64_t off = mxfp4a16_split_offset(P.M, P.K), left = a->scratch_bytes - off;
+    return launch_prefill(P, stream, stage, left > 0 ? P.scratch + off : nullptr, left > 0 ? left : 0);
+}
+
 static int entry(const RadArgs* a, RadStream s, int enc, bool decode) {
     if (enc == ENC_MXFP4A16 && env_no_mxfp4()) return RAD_E_UNSUPPORTED;
     if (enc == ENC_MXFP4A8 && (env_no_mxfp4() || (decode && env_no_fp4_dec())))
@@ -599,7 +606,7 @@ static int entry(const RadArgs* a, RadStream s, int enc, bool decode) {
     if (decode)
         return launch_decode(P, decode_splitk(a), stream, (uint8_t*)a->scratch,
                              a->scratch ? a->scratch_bytes : 0);
-    if (enc == ENC_MXFP4A16) return launch_prefill(P, stream);
+    if (enc == ENC_MXFP4A16) return launch_mxfp4a16(a, P, stream, 0);
     return launch_prefill(P, stream, 0, (uint8_t*)a->scratch, a->scratch ? a->scratch_bytes : 0);
 }
 
@@ -837,7 +844,9 @@ int64_t r3d_rad_gemm_nt_q_mxfp4a16_scratch(const RadArgs* a) {
     long long M = 0, K = 0;
     if (!rad_args_geti(a, "M", &M) || !rad_args_geti(a, "K", &K)) return 0;   /* 0 = none */
     if (M <= 0 || K <= 0 || M > (1LL << 27) || K > (1LL << 27)) return 0;
-    return r3d::mxfp4a16_scratch_bytes(M, K);
+    long long N = 0;                                     /* without N: the activations alone */
+    if (!rad_args_geti(a, "N", &N)) N = 0;
+    return r3d::mxfp4a16_hook_bytes(M, N, K, r3d::cu_count());
 }
 int r3d_rad_gemm_nt_q_fp8(const RadArgs* a, RadStream s) {
     return r3d::dump_wrap("gemm_nt_q_fp8a8", a, s, [](const RadArgs* x, RadStream t) {
@@ -870,7 +879,7 @@ int r3d_gfx950_mxfp4a16_stage(const RadArgs* a, RadStream s, int stage) {
     if (!r3d::chip_ok()) return RAD_E_UNSUPPORTED;
     /* the skinny band's decode-GEMV passes have no quantiser stage */
     if (r3d::skinny_passes(P.enc, P.M, P.N, r3d::cu_count())) return RAD_E_UNSUPPORTED;
-    return r3d::launch_prefill(P, (hipStream_t)s, stage);
+    return r3d::launch_mxfp4a16(a, P, (hipStream_t)s, stage);
 }
 
 }  /* extern "C" */

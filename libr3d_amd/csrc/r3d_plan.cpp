@@ -498,7 +498,7 @@ void prefill_geom(int64_t M, int64_t N, int64_t K, int mode, int ncu, PrefillGeo
     const bool narrow = mode == PF_F8 || (mode == PF_A8 && M <= 128);
     const int wmw = narrow ? 2 : 4;
     if (ncu <= 0) ncu = 256;
-    int best = 0;
+    int best = 0, best_m = wmw;
     double best_cost = 0.0;
     auto consider = [&](int w) {
         const int64_t tiles = ((N + 32 * w - 1) / (32 * w)) * ((M + 64 * wmw - 1) / (64 * wmw));
@@ -509,8 +509,15 @@ void prefill_geom(int64_t M, int64_t N, int64_t K, int mode, int ncu, PrefillGeo
         for (int w : kWnfF8) consider(w);
     else
         for (int w : kWnf) consider(w);
+    if (!narrow) {
+        /* e2m1 weights on 128 x 128: a round costs 2.85 fragment-steps (0.54 us a step against
+         * 0.87 of 128 x 256), so it runs where the larger tiles leave CUs idle (512 x 5376 x
+         * 5376: 168 tiles, 28 us, against 84 of 128 x 256, 41; at 714 tokens 30 against 42) */
+        const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128);
+        if ((double)((tiles + ncu - 1) / ncu) * 2.85 < best_cost) { best = 4; best_m = 2; }
+    }
     g->wnf = best;
-    g->wmf = wmw;
+    g->wmf = best_m;
     g->nst = 3;
     g->wv = 8;
     /* e4m3 weights past 128 tokens: four waves (one a SIMD, 512 registers each) hold a
@@ -640,6 +647,53 @@ int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, Prefil
     return (int)kbest;
 }
 
+/* The e2m1 tiles' K split past 128 tokens: the same fit over the mxfp4 rows' shapes (7 % mean
+ * error) -- a round of 128 x 128 and of 128 x 256, the wider tiles unsplit (w fragments: (w + 1/2)
+ * times 1000 + 193 a step), the planes and the reduce. */
+int prefill_mx_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g) {
+    if (M < kPrefillSplitM) return 0;
+    if (ncu <= 0) ncu = 256;
+    const int64_t steps = K / 128;
+    auto rounds = [&](int64_t tiles) { return (tiles + ncu - 1) / ncu; };
+    int64_t best = rounds(((N + 127) / 128) * ((M + 127) / 128)) * (2640 + 541 * steps);
+    for (int w : {8, 7, 6, 4}) {
+        const int64_t c = rounds(((N + 32 * w - 1) / (32 * w)) * ((M + 255) / 256)) * (2 * w + 1) *
+                          (500 + 193 * steps / 2);
+        if (c < best) best = c;
+    }
+    best = best * 88 / 100;          /* as prefill_f8_splitk's */
+    int64_t kbest = 0;
+    int mbest = 0;
+    for (int m = 2; m <= 4; m += 2) {
+        const int64_t tiles = ((N + 127) / 128) * ((M + 64 * m - 1) / (64 * m));
+        for (int64_t kc = 2; kc <= 32 && steps / kc >= 3 && tiles * kc <= 2 * ncu; ++kc) {
+            const int64_t cs = (steps + kc - 1) / kc, kk = (steps + cs - 1) / cs;
+            const int64_t bytes = kk * M * N * 4;
+            if (kk != kc || bytes > kPrefillSplitMaxBytes) continue;
+            const int64_t c = rounds(tiles * kk) * (m == 2 ? 2640 + 541 * cs : 4340 + 869 * cs) +
+                              5900 + bytes * 26 / 100000;
+            if (c < best) { best = c; kbest = kk; mbest = m; }
+        }
+    }
+    if (!kbest) return 0;
+    if (cst) *cst = (int)((steps + kbest - 1) / kbest);
+    if (g) {
+        *g = PrefillGeom{};
+        g->wnf = 4;
+        g->wmf = mbest;
+        g->nst = 3;
+        g->wv = 8;
+        g->bn = 128;
+        g->bm = 64 * mbest;
+        g->grid_n = (N + 127) / 128;
+        g->grid_m = (M + g->bm - 1) / g->bm;
+        g->tiles = g->grid_n * g->grid_m;
+        g->steps = (int)steps;
+        g->lds = g->nst * prefill_stage_bytes(4, mbest);
+    }
+    return (int)kbest;
+}
+
 int skinny_passes(int enc, int64_t M, int64_t N, int ncu) {
     if ((enc != ENC_MXFP4A8 && enc != ENC_FP8A8) || M < 17 || M > 64) return 0;
     static const int lever = [] {
@@ -721,13 +775,14 @@ static bool wide_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t kc0, Wid
 
 int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int* cst,
                 PrefillGeom* g, WideGeom* w) {
-    if (enc == ENC_FP8A8 && M > 128 && N > 0 && K >= 128) {
+    if (M > 128 && N > 0 && K >= 128) {
         int c = 0;
-        const int k = prefill_f8_splitk(M, N, K, ncu, &c, g);
+        const bool f8 = enc == ENC_FP8A8;
+        const int k = f8 ? prefill_f8_splitk(M, N, K, ncu, &c, g) : prefill_mx_splitk(M, N, K, ncu, &c, g);
         if (!k) return 0;
         if (kc) *kc = k;
         if (cst) *cst = c;
-        return 3;
+        return f8 ? 3 : 4;
     }
     if ((enc != ENC_MXFP4A8 && enc != ENC_FP8A8) || M < 1 || M > 128 || N < 1 || K < 128)
         return 0;
@@ -769,6 +824,17 @@ int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int*
 int64_t tile_splitk_bytes(int enc, int64_t M, int64_t N, int64_t K, int ncu) {
     int kc = 0;
     return splitk_plan(enc, M, N, K, ncu, &kc, nullptr, nullptr, nullptr) ? (int64_t)kc * M * N * 4 : 0;
+}
+
+int64_t mxfp4a16_split_offset(int64_t M, int64_t K) {
+    return (mxfp4a16_scratch_bytes(M, K) + 255) / 256 * 256;
+}
+
+int64_t mxfp4a16_hook_bytes(int64_t M, int64_t N, int64_t K, int ncu) {
+    const int64_t base = mxfp4a16_scratch_bytes(M, K);
+    if (M <= 128 || N <= 0 || N > kDimMax || base <= 0) return base;
+    const int64_t planes = tile_splitk_bytes(ENC_MXFP4A16, M, N, K, ncu);
+    return planes > 0 ? mxfp4a16_split_offset(M, K) + planes : base;
 }
 
 int64_t tile_scratch_bytes(const RadArgs* a, int enc, int ncu) {
@@ -1459,10 +1525,11 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
                  ename, (long long)P.M, (long long)P.N, (long long)P.K,
                  g.mt, g.chunks, g.waves, (long long)g.tiles, (long long)g.blocks, g.steps,
                  P.rblk);
-    } else if (int kc = 0, cst = 0, kind = a->scratch && ((uintptr_t)a->scratch & 15) == 0
+    } else if (int kc = 0, cst = 0, kind = a->scratch && ((uintptr_t)a->scratch & 15) == 0 && !P.ua
                                   ? splitk_plan(P.enc, P.M, P.N, P.K, 256, &kc, &cst, nullptr,
                                                 nullptr) : 0;
-               kind && a->scratch_bytes >= (int64_t)kc * P.M * P.N * 4) {
+               kind && a->scratch_bytes - (a16 ? mxfp4a16_split_offset(P.M, P.K) : 0) >=
+                           (int64_t)kc * P.M * P.N * 4) {
         PrefillGeom g{};
         WideGeom w{};
         splitk_plan(P.enc, P.M, P.N, P.K, 256, nullptr, nullptr, &g, &w);

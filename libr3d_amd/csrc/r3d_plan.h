@@ -210,6 +210,8 @@ int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu);
 constexpr int64_t kPrefillSplitM = 144;
 constexpr int64_t kPrefillSplitMaxBytes = int64_t(256) << 20;
 int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g);
+/* The e2m1 tiles' (128 x 128, 128 x 256) K split, from the same M; as prefill_f8_splitk. */
+int prefill_mx_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g);
 
 /* The skinny-band GEMV (gemv_wide_kernel, r3d_gemv_wide.h): 8 waves of tw 16-row weight
  * tiles (256 rows a workgroup at tw = 2) x one K chunk of cg groups; depth d lines in each
@@ -234,13 +236,17 @@ constexpr int kWideMaxLds = 152 * 1024;
 constexpr int kSplitMinSteps = 4;
 int tile_splitk(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g);
 /* The split's kernel: up to M = 64 the skinny-band GEMV (kind 1, *w), to 128 the 128 x 128
- * prefill tile (kind 2, *g), past that the fp8a8 wide tile (kind 3, *g); 0 when no split
- * applies.  *kc and *cst as tile_splitk's.
+ * prefill tile (kind 2, *g), past that the fp8a8 wide tile (kind 3, *g) or the e2m1 tiles
+ * (kind 4, *g; mxfp4a16 too); 0 when no split applies.  *kc and *cst as tile_splitk's.
  * R3D_GFX950_SPLITK_KERNEL=tile keeps the prefill tile (64 tokens a tile) up to M = 64. */
 int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int* cst,
                 PrefillGeom* g, WideGeom* w);
 /* Launch scratch the split needs: kc f32 planes of M x N (0 without a split). */
 int64_t tile_splitk_bytes(int enc, int64_t M, int64_t N, int64_t K, int ncu);
+/* The mxfp4a16 row: its split's planes follow the quantised activations, at this offset of the
+ * launch scratch, and its hook asks for both (the planes are optional, the activations not). */
+int64_t mxfp4a16_split_offset(int64_t M, int64_t K);
+int64_t mxfp4a16_hook_bytes(int64_t M, int64_t N, int64_t K, int ncu);
 /* The tile rows' scratch hook: tile_splitk_bytes at the args' N and K and M (numel(y) / N,
  * else the "M" param, else 128 -- the largest M the split takes); 0 without N or K. */
 int64_t tile_scratch_bytes(const RadArgs* a, int enc, int ncu);

@@ -37,7 +37,7 @@
  * VGPR needs two wait states before an MFMA reads it), and the accumulators are read
  * after the loop only past 24 further wait states (an 8-pass MFMA result needs 11 before
  * a VALU or v_accvgpr_read may read it).  Nothing else writes an accumulator, and each
- * accumulator is rewritten only once per K step, dozens of MFMAs apart.
+ * accumulator is rewritten only once per K step, eight or more MFMAs apart.
  */
 #ifndef R3D_PREFILL_H
 #define R3D_PREFILL_H
@@ -89,9 +89,9 @@ __global__ __launch_bounds__(64 * WV) void prefill_kernel(
      * major, weight tile fastest inside a group, so one round of 32 workgroups on an XCD
      * covers 8 weight x 4 token tiles (config 3: 10.3 MB of panels a round against 13.4 MB
      * for 4 x 8; measured 1-1.5 % faster). */
-    /* the split runs on the tiles of up to 128 tokens of the flushed modes only; the other
-     * instantiations compile it out (it costs them registers) and take kc = 1 */
-    constexpr bool KS = MODE != PF_MX8 && WMW <= 2 && WV == 8;
+    /* the split runs on the tiles of up to 128 tokens and, at e2m1 weights, on 128 x 256; the
+     * other instantiations compile it out (it costs them registers) and take kc = 1 */
+    constexpr bool KS = WV == 8 && (WMW <= 2 || (MODE != PF_F8 && WNF == 4));
     const int bid = blockIdx.x;
     const int units = KS ? tiles * kc : tiles;
     const int per = units >> 3, rem = units & 7, x = bid & 7;

@@ -145,8 +145,8 @@ F8_WIDE = [  # M, N, K, scratch: the fp8a8 wide tile, whole K and split
     (1030, 8448, 256, None),      # 256 x 256: two steps
     (300, 21700, 384, None),      # 256 x 128: an odd step count, ragged M and N
     (144, 300, 21504, "hook"),    # split: the least M, a ragged N past one tile
-    (500, 2050, 5376, "hook"),    # split, N off a multiple of 4
-    (513, 1000, 8192, "hook"),    # split, one live token in the last tile
+    (260, 514, 5376, "hook"),     # split, N off a multiple of 4
+    (513, 300, 8192, "hook"),     # split, one live token in the last tile
 ]
 
 
@@ -201,3 +201,64 @@ def test_fp8_wide_tile_non_finite_row_scale(gpu, bad):
     S8 = O.group8_mag("fp8a8", A, AS, B[rows], BS[rows], 1, nthreads=16)
     c = gu.compare(np.ascontiguousarray(Y[:, rows]), Yr, Yf, S, K, S8)
     assert c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0 and c["max_viol"] <= 1.0, c
+
+
+MX_SPLIT = [(144, 300, 8192), (260, 514, 5376), (513, 130, 6144)]   # M, N, K
+
+
+@pytest.mark.parametrize("M,N,K", MX_SPLIT)
+def test_mxfp4a8_prefill_splitk(gpu, M, N, K):
+    """K split past 128 tokens on the e2m1 tiles (ragged M and N, N off a multiple of 4, one
+    live token in the last tile), against the bar of the unsplit tiles; a scratch one byte
+    short runs those."""
+    gu = _gu()
+    A, AS, B, BS = _mx_case(M, N, K, M + N + K)
+    Yr, Yf, S = O.quant_dot_mxfp4a8(A, AS, B, BS, nthreads=16)
+    S8 = O.group8_mag("mxfp4a8", A, AS, B, BS, nthreads=16)
+    z = lambda *s, dt=torch.uint8: torch.zeros(s, dtype=dt)
+    ops = R.GemmOperands(z(M, K), z(M, K // 128, dt=torch.float32), z(N, K // 2), z(N, K // 32),
+                         z(M, N, dt=torch.int16), dtype="mxfp4a8", N=N, K=K)
+    need = R.row_scratch_bytes(MX_TILE, ops)
+    assert need > 0 and need % (4 * M * N) == 0
+    for scratch in ("hook", None):
+        rc, Y, guards = gu.run_row(MX_TILE, "mxfp4a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
+        assert rc == R.RAD_OK and guards
+        c = gu.compare(Y, Yr, Yf, S, K, S8)
+        assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
+        assert c["max_viol"] <= 1.0 and c["rel_l2"] <= 3e-2, c
+
+
+@pytest.mark.parametrize("M,N,K", MX_SPLIT)
+def test_mxfp4a16_prefill_splitk(gpu, M, N, K):
+    """The same on the bf16-in row, whose hook asks for the planes past the quantised
+    activations; with the activations' bytes alone, or one byte short of both, it runs
+    unsplit."""
+    gu = _gu()
+    X = _bf16_acts(M, K, M + N + K)
+    B, BS = synth.mxfp4_weights(N, K, M + 3)
+    Qr, SXr = O.quant_act_mxfp8(X)
+    Yr, Yf, S = O.dot_mx8_mxfp4(Qr, SXr, B, BS, nthreads=16)
+    S8 = O.group8_mag("mxfp4a16", Qr, SXr, B, BS, nthreads=16)
+    base = ((M * K + 255) // 256) * 256 + M * (K // 32)
+    gX, gB, gBS = gu.Guarded(X, gpu), gu.Guarded(B, gpu), gu.Guarded(BS, gpu)
+    for short in (None, 1, 0):                             # whole, one byte short, no planes
+        gY = gu.y_buffer(M, N, gpu)
+        ops = R.GemmOperands(gX.t, None, gB.t, gBS.t, gY.t, dtype="mxfp4a16", N=N, K=K, group=32,
+                             M=M)
+        need = R.row_scratch_bytes(A16, ops)
+        planes = need - (base + 255) // 256 * 256
+        assert planes > 0 and planes % (4 * M * N) == 0
+        nbytes = need if short is None else need - 1 if short else base
+        gS = gu.Guarded(np.zeros(nbytes, np.uint8), gpu, fill=0x5A)
+        ops.set_scratch(gS.t, nbytes)
+        arm = "arm=splitk" if short is None else "arm=prefill"
+        assert arm in R.describe(A16, ops)[1]
+        rc = R.launch_row(A16, ops, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == R.RAD_OK and all(g.guards_intact() for g in (gX, gB, gBS, gY, gS))
+        raw = gS.t.cpu().numpy()
+        assert np.array_equal(raw[:M * K].reshape(M, K), Qr)
+        Y = gY.t.cpu().numpy().view(np.uint16).reshape(M, N)
+        c = gu.compare(Y, Yr, Yf, S, K, S8)
+        assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
+        assert c["max_viol"] <= 1.0 and c["row_rel_l2_max"] <= 2.0 ** -8, c
