@@ -553,6 +553,123 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_fp8_kernel(
     }
 }
 
+/* The same for groups of 128 tiling rows of up to 8 T U values, every operand on its 16-byte
+ * walk: a lane keeps its U chunks of 8 values (chunk t + T u) in registers from the load to the
+ * codes, so the row passes through LDS once, for the sum of squares alone (lanes 0-255 walk it
+ * in the order above; values past n add +0, which changes no bit of a sum of squares), the
+ * weights are loaded with the row, and two barriers are left of five: every lane folds the
+ * eight half sums itself. */
+template <bool WBF16, int T, int U>
+__global__ __launch_bounds__(T) void rmsnorm_quant_fp8_reg_kernel(
+    const uint16_t* __restrict__ x, int64_t x_pitch, uint16_t* __restrict__ res, int64_t r_pitch,
+    const uint8_t* __restrict__ w, uint8_t* __restrict__ q, int64_t q_pitch,
+    float* __restrict__ sc, int64_t s_pitch, uint8_t* __restrict__ ob, int ob_bf16,
+    int64_t ob_pitch, int n, float eps, float wadd) {
+    __shared__ __attribute__((aligned(16))) uint16_t s_h[8 * T * U];
+    __shared__ float s_part[8];
+    const int t = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const uint16_t* xr = x + row * x_pitch;
+    uint16_t* rr = res ? res + row * r_pitch : nullptr;
+    auto bf = [](uint32_t b) { return __uint_as_float(b << 16); };
+    const int nc = n >> 3;
+    r3d_i32x4 v[U], a[U], wv[U][WBF16 ? 1 : 2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int c = t + T * u < nc ? t + T * u : nc - 1;
+        v[u] = *reinterpret_cast<const r3d_i32x4*>(xr + 8 * c);
+        if (rr) a[u] = *reinterpret_cast<const r3d_i32x4*>(rr + 8 * c);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int c = t + T * u < nc ? t + T * u : nc - 1;
+        wv[u][0] = *reinterpret_cast<const r3d_i32x4*>(w + (WBF16 ? 16 : 32) * c);
+        if (!WBF16) wv[u][WBF16 ? 0 : 1] = *reinterpret_cast<const r3d_i32x4*>(w + 32 * c + 16);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int c = t + T * u;
+        const bool in = c < nc;
+        if (rr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t lo = r3d_band_bf16_bits(__fadd_rn(
+                    bf((uint32_t)a[u][i] & 0xFFFFu), bf((uint32_t)v[u][i] & 0xFFFFu)));
+                const uint32_t hi = r3d_band_bf16_bits(__fadd_rn(bf((uint32_t)a[u][i] >> 16),
+                                                                 bf((uint32_t)v[u][i] >> 16)));
+                v[u][i] = (int)(lo | (hi << 16));
+            }
+            if (in) *reinterpret_cast<r3d_i32x4*>(rr + 8 * c) = v[u];
+        }
+        *reinterpret_cast<r3d_i32x4*>(s_h + 8 * c) = in ? v[u] : r3d_i32x4{0, 0, 0, 0};
+    }
+    __syncthreads();
+    if (t < 256) {
+        float ss = 0.0f;
+        constexpr int B = 8;                    /* reads in flight ahead of their adds */
+        for (int i0 = t; i0 < n; i0 += 256 * B) {
+            float e[B];
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                const int i = i0 + 256 * j;
+                e[j] = bf(i < 8 * T * U ? s_h[i] : 0u);
+            }
+#pragma unroll
+            for (int j = 0; j < B; ++j) ss = __fadd_rn(ss, __fmul_rn(e[j], e[j]));
+        }
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) ss = __fadd_rn(ss, __shfl_down(ss, off, 32));
+        if ((t & 31) == 0) s_part[t >> 5] = ss;
+    }
+    __syncthreads();
+    float r = s_part[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) r = __fadd_rn(r, s_part[k]);
+    const float rs = 1.0f / sqrtf(__fadd_rn(r / (float)n, eps));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int c = t + T * u;
+        if (T * u >= nc) break;                 /* whole workgroups: the shuffles below are whole */
+        float h[8];
+        r3d_i32x4 o;
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t b = (uint32_t)v[u][i >> 1] >> (16 * (i & 1)) & 0xFFFFu;
+            const float wf = WBF16 ? bf((uint32_t)wv[u][0][i >> 1] >> (16 * (i & 1)) & 0xFFFFu)
+                                   : __int_as_float(wv[u][WBF16 ? 0 : i >> 2][i & 3]);
+            const uint32_t hb = r3d_band_bf16_bits(
+                __fmul_rn(__fmul_rn(bf(b), rs), __fadd_rn(wf, wadd)));
+            h[i] = bf(hb);
+            if (i & 1) o[i >> 1] |= (int)(hb << 16);
+            else o[i >> 1] = (int)hb;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fmaxf(fabsf(h[2 * i]), fabsf(h[2 * i + 1])));
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        if (c >= nc) continue;
+        if (ob) {
+            if (ob_bf16) {
+                *reinterpret_cast<r3d_i32x4*>(ob + 2 * (row * ob_pitch + 8 * c)) = o;
+            } else {
+                float* of = reinterpret_cast<float*>(ob) + row * ob_pitch + 8 * c;
+                *reinterpret_cast<float4*>(of) = make_float4(h[0], h[1], h[2], h[3]);
+                *reinterpret_cast<float4*>(of + 4) = make_float4(h[4], h[5], h[6], h[7]);
+            }
+        }
+        const float s = amax > 0.0f ? amax * (1.0f / 448.0f) : 1.0f;
+        if ((c & 15) == 0) sc[row * s_pitch + (c >> 4)] = s;
+        const float inv = 1.0f / s;
+        float cv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) cv[i] = r3d_band_clamp448(h[i] * inv);
+        *reinterpret_cast<uint2*>(q + row * q_pitch + 8 * c) =
+            make_uint2(r3d_e4m3x4_rne(cv[0], cv[1], cv[2], cv[3]),
+                       r3d_e4m3x4_rne(cv[4], cv[5], cv[6], cv[7]));
+    }
+}
+
 }  // namespace r3d
 
 #endif /* R3D_BAND_H */

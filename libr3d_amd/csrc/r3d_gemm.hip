@@ -743,6 +743,33 @@ static int rms_entry(const RadArgs* a, RadStream s) {
     const bool vq = vec && P.g % 8 == 0 && lanes >= 1 && lanes <= 64 &&
                     (lanes & (lanes - 1)) == 0 && P.n % P.g == 0 &&
                     ((uintptr_t)P.q % 8) == 0 && P.q_pitch % 8 == 0;
+    /* groups of 128 on rows the registers of one workgroup hold: T lanes of U chunks.  Few rows
+     * (up to two a CU) leave the chip idle, so a row takes as many lanes as it has chunks; many
+     * rows want several resident a CU, so a lane takes two or three.  us, before -> after:
+     *   n = 5376   M = 4 7.0 -> 4.6 (1024, 1; the launch floor is 4.2), 256 8.1 -> 5.6,
+     *              2048 22.2 -> 21.0 (256, 3; 4.75 TB/s, a copy's rate; 1024 lanes 25.1)
+     *   n = 2304   M = 4 5.5 -> 4.1 (512, 1), 1024 9.0 -> 8.4; 4096 21.1, 21.9 at (512, 1): as it was
+     *   n = 8192   M = 4 9.0 -> 5.1 (1024, 1), 2048 33.1 -> 30.3 (512, 2)
+     *   n = 1024   M = 4 4.3 -> 4.2 (512, 1), 4096 13.5 -> 12.8 (256, 1) */
+    const int64_t nc = P.n / 8;
+    const bool few = P.rows <= 512;
+    const int shape = !vq || P.g != 128 ? 0
+                    : nc <= 256 ? (few ? 5121 : 2561)
+                    : nc <= 512 ? (P.rows <= 1536 ? 5121 : 0)
+                    : nc <= 768 ? (few ? 10241 : 2563)
+                    : nc <= 1024 ? (few ? 10241 : 5122)
+                    : nc <= 2048 && few ? 10242 : 0;
+#define R3D_RMR(W_, T_, U_)                                                                 \
+    hipLaunchKernelGGL((rmsnorm_quant_fp8_reg_kernel<W_, T_, U_>), dim3((unsigned)P.rows),    \
+                       dim3(T_), 0, stream, reinterpret_cast<const uint16_t*>(P.x), P.x_pitch, \
+                       reinterpret_cast<uint16_t*>(P.res), P.r_pitch, P.w, P.q, P.q_pitch,     \
+                       P.scale, P.s_pitch, P.ob, P.ob_bf16, P.ob_pitch, (int)P.n, P.eps, P.wadd)
+#define R3D_RMRS(W_)                                                                        \
+    switch (shape) {                                                                        \
+        case 2561: R3D_RMR(W_, 256, 1); break;   case 2563: R3D_RMR(W_, 256, 3); break;     \
+        case 5121: R3D_RMR(W_, 512, 1); break;   case 5122: R3D_RMR(W_, 512, 2); break;     \
+        case 10241: R3D_RMR(W_, 1024, 1); break; default: R3D_RMR(W_, 1024, 2); break;      \
+    }
 #define R3D_RMS(W_, V_, L_)                                                                 \
     hipLaunchKernelGGL((rmsnorm_quant_fp8_kernel<W_, V_, L_>), dim3((unsigned)P.rows),        \
                        dim3(256), lds, stream, reinterpret_cast<const uint16_t*>(P.x),        \
@@ -758,9 +785,13 @@ static int rms_entry(const RadArgs* a, RadStream s) {
         case 16: R3D_RMS(W_, true, 16); break; case 32: R3D_RMS(W_, true, 32); break;       \
         default: R3D_RMS(W_, true, 64); break;                                              \
     }
-    if (P.w_bf16) { R3D_RMSL(true) } else { R3D_RMSL(false) }
+    if (shape) {
+        if (P.w_bf16) { R3D_RMRS(true) } else { R3D_RMRS(false) }
+    } else if (P.w_bf16) { R3D_RMSL(true) } else { R3D_RMSL(false) }
 #undef R3D_RMSL
 #undef R3D_RMS
+#undef R3D_RMRS
+#undef R3D_RMR
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         fprintf(stderr, "libr3d_gfx950: rmsnorm_quant_fp8 launch FAILED (%s)\n", hipGetErrorName(e));

@@ -100,3 +100,24 @@ def test_rmsnorm_quant_special_values(gpu):
     _check(x, w, gpu)
     r = synth.bf16_bits(rng.standard_normal((4, 1024)).astype(np.float32))
     _check(x, w, gpu, residual=r)
+
+
+@pytest.mark.parametrize("M,n", [(3, 128), (513, 256), (2, 2048), (3, 2176), (1536, 2176), (2, 4096),
+                                 (512, 4224), (513, 4224), (520, 6144), (4, 6272), (530, 6272),
+                                 (3, 8192), (2, 8320), (2, 16384)])
+@pytest.mark.parametrize("form", ["bare", "full"])
+def test_register_rows(gpu, M, n, form):
+    """Rows held in registers, at both ends of every (lanes, chunks) shape: one row in memory
+    fewer or more lanes than chunks, and one workgroup of each row count's rule; bare (f32 w, no
+    residual, no output) and full (bf16 w, residual, wadd, f32 output); a NaN, an Inf and an
+    all-zero row among them."""
+    print("rmsnorm register rows M=%d n=%d %s" % (M, n, form), flush=True)
+    x, rng = _x(M, n, M + n)
+    x[0, 5], x[1, n - 1], x[M - 1, :] = 0x7FC0, 0x7F80, 0
+    w = (1 + 0.2 * rng.standard_normal(n)).astype(np.float32)
+    if form == "bare":
+        _check(x, w, gpu, out=None)
+    else:
+        r, _ = _x(M, n, 7 * M + n)
+        r[M - 1, :] = 0
+        _check(x, synth.bf16_bits(w), gpu, wadd=1.0, residual=r, out="f32")
