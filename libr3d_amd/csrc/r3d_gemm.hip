@@ -142,21 +142,25 @@ static int launch_lines(const GemmPlan& P, const LinesGeom& g, hipStream_t strea
                         int passes = 1) {
     if (forced_fail(passes > 1 ? "skinny" : "lines"))
         return launch_failed(passes > 1 ? "skinny line GEMV" : "line decode GEMV", hipSuccess);
-    const dim3 grid((unsigned)g.blocks, (unsigned)passes), block(256);
+    const dim3 grid((unsigned)g.blocks, (unsigned)passes), block((unsigned)(64 * g.wv));
     const int64_t lim = (int64_t)1 << 31;
-    if (P.M < 1 || P.M > 127 || (g.chunks != 1 && g.chunks != 2 && g.chunks != 4) ||
+    int cl = 0;
+    while (cl < 3 && (1 << cl) < g.chunks) ++cl;
+    if (P.M < 1 || P.M > 127 || g.chunks != 1 << cl || g.wv != (cl == 3 ? 8 : 4) ||
+        (g.wv == 8 && g.tw != 1) ||
         P.a_pitch >= lim || P.as_pitch >= lim || P.b_pitch >= lim || P.bs_pitch >= lim ||
         g.wlds != lines_wlds(P.enc, g.tw, P.K, g.chunks))
         return RAD_E_UNSUPPORTED;
-    const int pk = lines_pack((int)P.M, g.chunks == 4 ? 2 : g.chunks == 2 ? 1 : 0, P.rblk == 128,
-                              P.as_pitch == P.K / 128);
-#define R3D_LINES(ENC_, MT_, TW_, D_)                                                        \
-    hipLaunchKernelGGL((gemv_lines_kernel<ENC_, MT_, TW_, D_>), grid, block, (size_t)g.lds,    \
+    const int pk = lines_pack((int)P.M, cl, P.rblk == 128, P.as_pitch == P.K / 128);
+#define R3D_LINES(ENC_, MT_, TW_, D_) R3D_LINESW(ENC_, MT_, TW_, D_, 4)
+#define R3D_LINESW(ENC_, MT_, TW_, D_, WV_)                                                  \
+    hipLaunchKernelGGL((gemv_lines_kernel<ENC_, MT_, TW_, D_, WV_>), grid, block, (size_t)g.lds, \
                        stream, P.A, P.AS, P.B, P.BS, (int)P.N, (int)P.K, (int)P.b_pitch,     \
                        (int)P.bs_pitch, (int)P.a_pitch, pk, (int)P.as_pitch, P.Y, P.y_pitch)
 #define R3D_LINES_T(ENC_, MT_, D_)                                                           \
     do {                                                                                     \
-        if (g.tw == 4) R3D_LINES(ENC_, MT_, 4, (D_ > 2 ? 2 : D_));                           \
+        if (g.wv == 8) R3D_LINESW(ENC_, MT_, 1, (D_ > 2 ? 2 : D_), 8);                  \
+        else if (g.tw == 4) R3D_LINES(ENC_, MT_, 4, (D_ > 2 ? 2 : D_));                      \
         else if (g.tw == 2) R3D_LINES(ENC_, MT_, 2, D_);                                     \
         else R3D_LINES(ENC_, MT_, 1, D_);                                                    \
     } while (0)
@@ -178,6 +182,7 @@ static int launch_lines(const GemmPlan& P, const LinesGeom& g, hipStream_t strea
 #undef R3D_LINES_T
 #undef R3D_LINES_D
 #undef R3D_LINES
+#undef R3D_LINESW
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return launch_failed("line decode GEMV", e);
     debug_once(P.enc == ENC_MXFP4A8 ? "mxfp4a8 line decode GEMV" : "fp8a8 line decode GEMV",

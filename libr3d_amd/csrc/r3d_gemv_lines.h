@@ -7,19 +7,19 @@
  * so every product of the MFMA is used.  The unit of the walk is a LINE: 128 contiguous
  * bytes of every weight row -- one 128-wide K group at fp8a8, two at mxfp4a8 (64 bytes of
  * e2m1 codes per group).  A wave fetches a unit with two buffer_load_dwordx4, the first
- * covering rows 0-7 and the second rows 8-15, each in whole 128-byte lines (an
- * instruction walking all 16 rows could only cover half lines, which streams ~25 % slower
- * on MI355X).  The activation rows of each group arrive the same way (rows 0-7, rows
- * 8-15) straight into registers, from L2: at M = 16 they are as many bytes per group as
- * the weights, far too many to stage whole in LDS, and every wave reads them in the same
- * order as its weights.
+ * covering rows 0-7 and the second rows 8-15: lane l of a load holds chunk l % 8 of row l / 8,
+ * so eight lanes in a row read one whole 128-byte line.  The activation rows of each group
+ * arrive the same way (rows 0-7, rows 8-15) straight into registers, from L2: at M = 16 they
+ * are as many bytes per group as the weights, far too many to stage whole in LDS, and every
+ * wave reads them in the same order as its weights.
  *
- * Register shuffle.  Inside one 16-lane row of the wave, the first load gives lane p the
- * 16-byte chunk ca = kb (p < 8) or 4 + kb (p >= 8) of row p % 8, and the second load the
- * chunk cb = 4 + kb (p < 8) or kb (p >= 8) of row 8 + p % 8 (kb = lane / 16).  Then
- *     lo = (p < 8 ? load0 : load1)            -> row p, chunk kb
- *     hi = row_ror:8 of (p < 8 ? load1 : load0) -> row p, chunk 4 + kb
- * (one select and two DPP rotates per register).  For an fp8 operand (lo,
+ * The MFMA wants lane 16 kb + p to hold row p's chunks kb (lo) and 4 + kb (hi).  The two loads
+ * take that form through 2 KB of the wave's own LDS (r3d_lines_turn).  Loading them in it
+ * directly (each lane its own row, a select and two DPP rotates per register) takes the address
+ * unit a row a lane: about 64 clocks a KB, which bounded a workgroup at 16 bytes a clock however
+ * few of them ran (512 x 17152 at M = 14: 19.4 us e2m1 and 25.1 e4m3, 13.5 and 19.4 turned).
+ *
+ * For an fp8 operand (lo,
  * hi) are exactly the MFMA's bytes [16kb, +16) and [64 + 16kb, +16) of the lane's row;
  * for e2m1 weights lo is the lane's 32-wide block of the line's first group and hi that of
  * the second.  The per-group sums are then libref's per-group subs: the a_scale (and the
@@ -32,7 +32,8 @@
  * weight scales (mxfp4a8: [16 rows][gmax] E8M0 dwords; fp8a8: [gmax][16 rows] 4-byte
  * slots, bf16 in the low half) in its wlds-byte slice of LDS, then primes the ring.
  *
- * Work split: a workgroup is 4 waves = (4 / chunks) tiles x chunks; the chunks of a tile
+ * Work split: a workgroup is 4 waves = (4 / chunks) tiles x chunks, or 8 waves, all chunks of
+ * one tile, where few rows and a long K leave the chip idle (lines_geom); the chunks of a tile
  * fold through LDS in a fixed order (deterministic).  Rows past N clamp to row N-1,
  * activation rows past M duplicate row M-1, groups past a chunk clamp to its last group;
  * none of these is accumulated or stored. */
@@ -58,6 +59,19 @@ __device__ __forceinline__ void r3d_lines_fix(const r3d_i32x4& a, const r3d_i32x
     }
 }
 
+/* (lo, hi) operand registers of 16 rows from their two loads (lane l of load h: row 8 h + l / 8,
+ * chunk l % 8), through 2 KB of the wave's own LDS: row r's chunk c sits at
+ * 128 r + 16 (c ^ r % 8), so eight lanes writing a row and eight lanes reading one chunk of
+ * eight rows both cover eight distinct 16-byte banks.  A wave's LDS operations run in order, so
+ * the next tile may follow in the same 2 KB at once. */
+__device__ __forceinline__ void r3d_lines_turn(uint8_t* buf, int wr, int rd, const r3d_i32x4& a,
+                                               const r3d_i32x4& b, r3d_i32x4& lo, r3d_i32x4& hi) {
+    *reinterpret_cast<r3d_i32x4*>(buf + wr) = a;
+    *reinterpret_cast<r3d_i32x4*>(buf + 1024 + wr) = b;
+    lo = *reinterpret_cast<const r3d_i32x4*>(buf + rd);
+    hi = *reinterpret_cast<const r3d_i32x4*>(buf + (rd ^ 64));
+}
+
 /* One unit of one wave in the ring: the line pairs of its TW weight tiles and, per group of
  * the unit, the activation pair (only the rows 0-7 load when MT is 8). */
 template <int ENC, int MT, int TW>
@@ -69,18 +83,18 @@ struct LinesUnit {
 };
 
 /* The small parameters packed into one argument: M (1..64: the skinny band's passes see
- * up to 16 each) in bits 0-6, log2 of the chunk count (0..2) in bits 7-8, fp8a8 weight
- * scales on the 128 x 128 block grid in bit 9, a_scale rows at a pitch of K / 128 floats
- * in bit 10. */
+ * up to 16 each) in bits 0-6, log2 of the chunk count (0..4) in bits 7-9, fp8a8 weight
+ * scales on the 128 x 128 block grid in bit 10, a_scale rows at a pitch of K / 128 floats
+ * in bit 11. */
 constexpr int lines_pack(int M, int log2_chunks, bool rblk128, bool as_dense) {
-    return M | (log2_chunks << 7) | ((int)rblk128 << 9) | ((int)as_dense << 10);
+    return M | (log2_chunks << 7) | ((int)rblk128 << 10) | ((int)as_dense << 11);
 }
 
 /* The arguments the prologue needs come first (the hardware preloads the leading 14 dwords
  * of the argument block at dispatch); as_pitch (rows not dense), Y and its pitch follow.
  * Pitches in bytes (b, a), bf16 / E8M0 elements (bs) or floats (as), below 2^31. */
-template <int ENC, int MT, int TW, int D>
-__global__ __launch_bounds__(256) void gemv_lines_kernel(
+template <int ENC, int MT, int TW, int D, int WV = 4>
+__global__ __launch_bounds__(64 * WV) void gemv_lines_kernel(
     const uint8_t* A, const float* AS, const uint8_t* B, const void* BSv,
     int N, int K, int b_pitch, int bs_pitch, int a_pitch, int pk,
     int as_pitch, uint16_t* __restrict__ Y, int64_t y_pitch) {
@@ -89,8 +103,8 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
     constexpr int RW = 16 * TW;                            /* weight rows per wave */
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int M = pk & 127;
-    const int cl = (pk >> 7) & 3, chunks = 1 << cl;
-    const bool rblk128 = (pk >> 9) & 1, as_dense = (pk >> 10) & 1;
+    const int cl = (pk >> 7) & 7, chunks = 1 << cl;
+    const bool rblk128 = (pk >> 10) & 1, as_dense = (pk >> 11) & 1;
     const int groups = K >> 7;
     /* grid.y > 1 (the skinny band): workgroup row y computes activation rows
      * [16 y, 16 y + 16) of a taller A -- the same arithmetic as a 16-row call (AS moves
@@ -105,7 +119,7 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int units = (groups + G - 1) / G;
-    const int tpb = 4 >> cl;                               /* row blocks per workgroup */
+    const int tpb = WV >> cl;                              /* row blocks per workgroup */
     const int ti = wave >> cl, c = wave & (chunks - 1);
     const int64_t n0 = ((int64_t)blockIdx.x * tpb + ti) * RW;
     const int u0 = (units * c) >> cl;                      /* units < 2^21: no overflow */
@@ -117,9 +131,7 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
     const int gc = (G * ns < groups - g0) ? G * ns : groups - g0;   /* real groups */
 
     const int p = lane & 15;           /* row of src A / column of src B inside a tile */
-    const bool first = p < 8;
     const int kb = lane >> 4;
-    const int r8 = lane & 7;
 
     /* ---- 1. LDS staging of this wave's scales: a_scales [16][gmax] f32 in the first xsb
      * bytes of its slice, then the weight scales of its RW rows */
@@ -173,18 +185,20 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
         const_cast<uint8_t*>(B + n0 * b_pitch), (short)0, (int)(rows * b_pitch), 0x00020000);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(A), (short)0, (int)((int64_t)(M - 1) * a_pitch + K), 0x00020000);
-    const int ca = p < 8 ? kb : 4 + kb, cb = p < 8 ? 4 + kb : kb;
+    const int lr = lane >> 3, lc = lane & 7;               /* a load's row and chunk of this lane */
+    uint8_t* const turn = smem + WV * wlds + kLinesTurn * wave;
+    const int twr = 128 * lr + 16 * (lc ^ lr), trd = 128 * p + 16 * (kb ^ (p & 7));
     uint32_t wa[TW], wb[TW];
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
-        const int64_t ra = n0 + 16 * t + r8 < N ? n0 + 16 * t + r8 : N - 1;
-        const int64_t rb = n0 + 16 * t + 8 + r8 < N ? n0 + 16 * t + 8 + r8 : N - 1;
-        wa[t] = (uint32_t)((ra - n0) * b_pitch + 16 * ca);
-        wb[t] = (uint32_t)((rb - n0) * b_pitch + 16 * cb);
+        const int64_t ra = n0 + 16 * t + lr < N ? n0 + 16 * t + lr : N - 1;
+        const int64_t rb = n0 + 16 * t + 8 + lr < N ? n0 + 16 * t + 8 + lr : N - 1;
+        wa[t] = (uint32_t)((ra - n0) * b_pitch + 16 * lc);
+        wb[t] = (uint32_t)((rb - n0) * b_pitch + 16 * lc);
     }
-    const int ta = r8 < M ? r8 : M - 1, tb = 8 + r8 < M ? 8 + r8 : M - 1;
-    const uint32_t xa = (uint32_t)(ta * a_pitch + 16 * ca);
-    const uint32_t xb = (uint32_t)(tb * a_pitch + 16 * cb);
+    const int ta = lr < M ? lr : M - 1, tb = 8 + lr < M ? 8 + lr : M - 1;
+    const uint32_t xa = (uint32_t)(ta * a_pitch + 16 * lc);
+    const uint32_t xb = (uint32_t)(tb * a_pitch + 16 * lc);
 
     using Unit = LinesUnit<ENC, MT, TW>;
     const uint32_t kSkip = 0x80000000u;
@@ -238,21 +252,20 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
     auto consume = [&](const Unit& v, int s) {
         r3d_i32x4 wlo[TW], whi[TW];
 #pragma unroll
-        for (int t = 0; t < TW; ++t) r3d_lines_fix(v.w0[t], v.w1[t], first, wlo[t], whi[t]);
+        for (int t = 0; t < TW; ++t) r3d_lines_turn(turn, twr, trd, v.w0[t], v.w1[t], wlo[t], whi[t]);
 #pragma unroll
         for (int h = 0; h < G; ++h) {
             const int gl = G * s + h;                      /* group inside the chunk */
             const bool live = gl < gc;
             const int gr = live ? gl : gc - 1;
             r3d_i32x4 xlo, xhi;
-            if (MT == 16) {
-                r3d_lines_fix(v.x0[h], v.x1[h], first, xlo, xhi);
+            if constexpr (MT == 16) {
+                r3d_lines_turn(turn, twr, trd, v.x0[h], v.x1[h], xlo, xhi);
             } else {
-                /* columns 8-15 of the result are never stored: only rows p < 8 of B matter */
-                xlo = v.x0[h];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    xhi[i] = __builtin_amdgcn_mov_dpp(v.x0[h][i], 0x128, 0xF, 0xF, false);
+                /* result columns 8-15 are never stored: rows 0-7 stand in for them */
+                *reinterpret_cast<r3d_i32x4*>(turn + twr) = v.x0[h];
+                xlo = *reinterpret_cast<const r3d_i32x4*>(turn + (trd & 1023));
+                xhi = *reinterpret_cast<const r3d_i32x4*>(turn + ((trd & 1023) ^ 64));
             }
             const r3d_i32x8 bv = {xlo[0], xlo[1], xlo[2], xlo[3], xhi[0], xhi[1], xhi[2], xhi[3]};
             const float a_s = xs[gr];
@@ -311,7 +324,7 @@ __global__ __launch_bounds__(256) void gemv_lines_kernel(
     for (int t = 0; t < TW; ++t) red[(wave * TW + t) * 64 + lane] = acc[t];
     __syncthreads();
     const float* rf = reinterpret_cast<const float*>(smem);
-    for (int o = threadIdx.x; o < tpb * RW * MT; o += 256) {
+    for (int o = threadIdx.x; o < tpb * RW * MT; o += 64 * WV) {
         const int r = o % RW, tk = (o / RW) % MT, b = o / (RW * MT);
         const int t = r >> 4, rr = r & 15;
         float y = 0.0f;

@@ -437,15 +437,34 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
     g->groups = (int)(K / 128);
     g->units = (g->groups + G - 1) / G;
     g->tiles = (N + 15) / 16;
-    /* two tiles per wave halve the activation loads per weight byte; measured best on
-     * MI355X at the 27B-class shapes (M = 8..16) */
+    /* On a small launch a wave's own chain of turns and MFMAs bounds the time and one tile per
+     * wave is best; on a large one two tiles, which halve the activation bytes per weight byte.
+     * Measured on MI355X at M = 14 (us, one tile and two): e2m1 512 x 5376 4.9 6.3, 5376 x 2560
+     * 5.6 7.1, 8192 x 5376 8.1 8.3, 5120 x 10624 13.9 13.2, 21504 x 5376 19.1 17.6; e4m3
+     * 2304 x 5376 7.0 9.1, 5120 x 10624 16.4 15.5, 21504 x 5376 24.2 21.6.  Past 768 tiles the
+     * waves of one tile no longer fit the chip at once, unless K is short (e2m1 16384 x 2560 9.7
+     * 8.0, 15104 x 1920 8.7 7.2, 21504 x 1536 7.6 8.7); up to 256 tiles the split in 8 below needs one.  With 8
+     * activation rows e2m1 loads half as many activation bytes and keeps one tile up to 2^26
+     * weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4). */
     const int etw = env_lines_tw();
-    g->tw = etw == 1 || etw == 2 || etw == 4 ? etw : 2;
+    const bool small = g->tiles <= 256 ||
+                       (enc == ENC_MXFP4A8 && g->mt == 8
+                            ? N * K < ((int64_t)1 << 26)
+                            : N * K < ((int64_t)45 << 20) && (g->tiles <= 768 || K < 1920));
+    g->tw = etw == 1 || etw == 2 || etw == 4 ? etw : small ? 1 : 2;
     g->nblk = (g->tiles + g->tw - 1) / g->tw;
     auto wlds_of = [&](int c) { return lines_wlds(enc, g->tw, K, c); };
     int c = 1;
     if (force_chunks > 0) {
         c = (int)force_chunks;
+    } else if (g->tw == 1) {
+        /* One tile: the time goes with the units of a wave, so K is cut in 4 as soon as that
+         * leaves a unit each (2304 x 1152 at M = 14, 2 -> 4 chunks: e2m1 4.7 -> 4.5, e4m3
+         * 5.0 -> 4.5; below 512 rows from the ninth unit on), and in 8 where every tile still
+         * has a CU to itself and two units a wave (4 -> 8: e4m3 2304 x 2560 5.0 -> 4.7,
+         * 512 x 17152 14.2 -> 12.1; 16 chunks give no more). */
+        c = g->units >= (g->tiles < 32 ? 9 : 4) ? 4 : g->units >= 2 ? 2 : 1;
+        if (g->units >= 16 && g->tiles <= 256) c = 8;
     } else {
         const int64_t target = env_lines_waves();
         while (c < 4 && g->units >= 8 * c &&
@@ -454,23 +473,25 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
     }
     while (c > 1 && c > g->units) c >>= 1;
     g->chunks = c;
-    g->tpb = 4 / c;
+    g->wv = c == 8 ? 8 : 4;
+    g->tpb = g->wv / c;
     g->blocks = (g->nblk + g->tpb - 1) / g->tpb;
     g->gmax = G * ((g->units + c - 1) / c);
     g->wlds = wlds_of(c);
-    const int fold = 4 * 1024 * g->tw;
-    g->lds = 4 * g->wlds > fold ? 4 * g->wlds : fold;
+    const int fold = g->wv * 1024 * g->tw;
+    g->lds = g->wv * (g->wlds + kLinesTurn);
+    if (g->lds < fold) g->lds = fold;
     {
         static const int kDepths[] = {4, 2, 1};
         const int ns_min = g->units / c;
         const int ed = env_lines_depth();
-        int want = ed > 0 ? ed : (g->tw >= 2 ? 2 : 4);   /* measured best */
+        int want = ed > 0 ? ed : 2;                       /* measured best */
         if (g->tw >= 4 && want > 2) want = 2;             /* register budget */
         g->depth = 1;
         for (int d : kDepths)
             if (d <= want && d <= ns_min) { g->depth = d; break; }
     }
-    return g->lds <= kLinesMaxLds && g->blocks <= 0x7FFFFFFF;
+    return g->wlds <= kLinesMaxLds / 4 && g->blocks <= 0x7FFFFFFF;
 }
 
 /* Prefill tile choice: 64 wmw tokens (4 fragments per wave; 2 with e4m3 weights, whose
@@ -1511,9 +1532,9 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
     } else if (LinesGeom lg{}; dec && lines_fits(P) &&
                lines_geom(P.enc, P.M, P.N, P.K, decode_splitk(a), &lg)) {
         snprintf(buf, (size_t)len,
-                 "arm=decode kernel=lines enc=%s M=%lld N=%lld K=%lld mt=%d tw=%d chunks=%d waves=4 "
+                 "arm=decode kernel=lines enc=%s M=%lld N=%lld K=%lld mt=%d tw=%d chunks=%d waves=%d "
                  "tiles=%lld blocks=%lld units=%d depth=%d lds=%d rblk=%d",
-                 ename, (long long)P.M, (long long)P.N, (long long)P.K, lg.mt, lg.tw, lg.chunks,
+                 ename, (long long)P.M, (long long)P.N, (long long)P.K, lg.mt, lg.tw, lg.chunks, lg.wv,
                  (long long)lg.tiles, (long long)lg.blocks, lg.units, lg.depth, lg.lds, P.rblk);
     } else if (dec) {
         DecodeGeom g{};

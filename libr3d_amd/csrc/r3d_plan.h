@@ -103,8 +103,8 @@ constexpr QuadLds quad_lds(int enc, int mt, int qpw, int wv, int64_t K, int chun
 }
 
 /* The line GEMV's per-wave LDS slice (a_scales [16][gmax] f32, then the weight scales of
- * its 16 tw rows over gmax groups, each rounded up to 256 B) for `chunks` (1, 2 or 4) K
- * chunks; the kernel computes it the same way. */
+ * its 16 tw rows over gmax groups, each rounded up to 256 B) for `chunks` (1, 2, 4 or 8)
+ * K chunks; the kernel computes it the same way. */
 constexpr int lines_wlds(int enc, int tw, int64_t K, int chunks) {
     const int G = enc == ENC_MXFP4A8 ? 2 : 1;
     const int units = (int)(((K >> 7) + G - 1) / G);
@@ -113,13 +113,14 @@ constexpr int lines_wlds(int enc, int tw, int64_t K, int chunks) {
 }
 
 /* Launch geometry of the line GEMV (M <= 16): one wave per block of tw 16-row weight tiles
- * and K chunk, 4 waves per workgroup (4 / chunks blocks x chunks); a unit is one 128-byte
- * line of every row of the block (2 K groups at mxfp4a8, 1 at fp8a8). */
+ * and K chunk, 4 waves per workgroup (4 / chunks blocks x chunks), or 8 waves at 8 chunks; a
+ * unit is one 128-byte line of every row of the block (2 K groups at mxfp4a8, 1 at fp8a8). */
 struct LinesGeom {
     int mt;                  /* activation rows of the instantiation: 8 or 16 */
     int tw;                  /* 16-row tiles per wave: 1, 2 or 4 */
-    int chunks;              /* waves per row block (split-K): 1, 2 or 4 */
-    int tpb;                 /* row blocks (16 tw rows) per workgroup: 4 / chunks */
+    int chunks;              /* waves per row block (split-K): 1, 2, 4 or 8 */
+    int wv;                  /* waves per workgroup: 4, or 8 at 8 chunks */
+    int tpb;                 /* row blocks (16 tw rows) per workgroup: wv / chunks */
     int groups, units;       /* K / 128; lines per row */
     int gmax;                /* most K groups one chunk holds */
     int depth;               /* ring depth in units (<= every wave's unit count) */
@@ -175,7 +176,8 @@ bool quad_fits(const GemmPlan& P);
 /* Line GEMV geometry; false when the shape is outside what it serves (M outside 5..16, or a
  * wave's scale tables over the LDS budget), and the 16-row GEMV runs instead.  force_chunks:
  * 1/2/4 pin the split, anything else above 0 leaves the line kernel. */
-constexpr int kLinesMaxLds = 48 * 1024;
+constexpr int kLinesMaxLds = 48 * 1024;     /* scale tables of 4 waves */
+constexpr int kLinesTurn = 2048;            /* a wave's LDS for turning loads into operands */
 bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, LinesGeom* g);
 /* The line kernel addresses a wave's (up to 64) weight rows and the whole activation plane through
  * buffer resources: both must span less than 2^31 bytes. */

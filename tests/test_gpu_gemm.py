@@ -133,6 +133,26 @@ def test_fp8_decode_lines_shapes(gpu, N, K, M, rblk):
     _check(F8_DEC, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk)
 
 
+@pytest.mark.parametrize("M", [5, 8, 9, 16])
+@pytest.mark.parametrize("dtype,N,K,geom", [
+    # the smallest K of 4 and of 8 chunks, a ragged last tile, an odd group count (half a line
+    # at e2m1), both sides of the 256 tiles that 8 chunks take and of one and two tiles a wave
+    ("mxfp4a8", 500, 896, (1, 4)), ("mxfp4a8", 500, 3968, (1, 8)), ("mxfp4a8", 4096, 3840, (1, 4)),
+    ("mxfp4a8", 4112, 4096, (1, 4)), ("mxfp4a8", 12305, 5504, (2, 4)),
+    ("mxfp4a8", 12305, 1152, (1, 4)),
+    ("fp8a8", 515, 512, (1, 4)), ("fp8a8", 4095, 2048, (1, 8)), ("fp8a8", 4097, 2048, (1, 4)),
+    ("fp8a8", 33, 1152, (1, 4)), ("fp8a8", 12305, 2176, (2, 4))])
+def test_decode_lines_split_rule(gpu, dtype, N, K, geom, M):
+    row = MX_DEC if dtype == "mxfp4a8" else F8_DEC
+    A, AS, B, BS = (_mx_case(M, N, K, M + N + K) if dtype == "mxfp4a8"
+                    else _f8_case(M, N, K, M + N + K, 1))
+    from tests.test_abi import _f8_ops, _mx_ops
+    ops = (_mx_ops if dtype == "mxfp4a8" else _f8_ops)(M=M, N=N, K=K)[0]
+    d = R.describe(row, ops)[1]
+    assert "kernel=lines" in d and "tw=%d chunks=%d" % geom in d, d
+    _check(row, dtype, A, AS, B, BS, M, N, K, gpu)
+
+
 @pytest.mark.parametrize("pad,offset", [(4, 0), (0, 4), (12, 8)])
 def test_mxfp4_decode_scale_plane_layouts(gpu, pad, offset):
     """The E8M0 plane as a padded-pitch and/or 4-byte (not 16-byte) aligned view: the decode
