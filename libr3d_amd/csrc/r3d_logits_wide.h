@@ -4,9 +4,10 @@
  * A workgroup of 8 waves owns blocks of 128 TW head rows (a wave TW tiles of 16), each over
  * the whole of K in 256-wide windows, as one stream of windows across its blocks.  The codes
  * arrive in whole 128-byte lines straight into registers, one window ahead (two loads per
- * 16 rows x 128 bytes, rows 0-7 and 8-15, put in operand order by one select and two DPP
- * rotates, r3d_lines_fix): lane 16 kb + p then holds head row p's 16-byte chunks kb and 4 + kb
- * of a line -- one 128-wide scale block -- which widen exactly to the operands of four
+ * 16 rows x 128 bytes, rows 0-7 and 8-15, eight lanes a line, put in operand order through 2 KB
+ * of the wave's LDS, r3d_lines_turn; a load of a row a lane with the shuffle in registers takes
+ * 242 us where this takes 228): lane 16 kb + p then holds head row p's 16-byte chunks kb and
+ * 4 + kb of a line -- one 128-wide scale block -- which widen exactly to the operands of four
  * v_mfma_f32_16x16x32_bf16.  All 16 columns of the MFMA are activation rows, against the 4 of
  * 16 products that the 4-row walk uses.  A window's activation rows (16 NTG of them, zero past
  * M and past K) sit in LDS, double-buffered, XOR-swizzled by row so that eight lanes reading
@@ -16,14 +17,15 @@
  *
  * Bound: the head's bytes from HBM.  262144 x 5376 (1.43 GB), bf16 scale per row x 128, us:
  *
- *   M                      12    16    32    64
- *   8-row passes          464   475   949  1899
- *   this walk, TW = 2     237   243   259   321
- *   this walk, TW = 1     254   260   290   371
+ *   M                                     16    32    64
+ *   8-row passes                         475   949  1899
+ *   a row a lane, TW = 1                 260   290   371
+ *   a row a lane, TW = 2                 243   259   321
+ *   this walk (eight lanes a line), TW 2 228   243   316
  *
  * TW = 1 restages the activation rows twice as often per head row but balances twice as
- * finely over the workgroups (151936 x 4096, M = 16: 132 against 146 us; 32000 x 4096: 31
- * against 42); logits_wide_tiles picks.  Measured without gain: three windows of codes in
+ * finely over the workgroups (151936 x 4096, M = 16: 132 against 146 us with a row a lane, 122
+ * now; 32000 x 4096: 31 against 42); logits_wide_tiles picks.  Measured without gain: three windows of codes in
  * flight (TW = 1: 262 us), four waves a workgroup (293), sixteen (spills). */
 #ifndef R3D_LOGITS_WIDE_H
 #define R3D_LOGITS_WIDE_H
@@ -44,8 +46,7 @@ void logits_wide_kernel(
     static_assert(TW <= 2, "one scale load covers a window's tiles");
     extern __shared__ __align__(16) uint8_t lg_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l = threadIdx.x & 63, p = l & 15, kb = l >> 4, r8 = l & 7;
-    const bool first = p < 8;
+    const int l = threadIdx.x & 63, p = l & 15, kb = l >> 4;
     const int mb = blockIdx.y * 64;
     const int live = M - mb < 16 * NTG ? M - mb : 16 * NTG;
     const int blocks = (N + RB - 1) / RB;
@@ -69,7 +70,10 @@ void logits_wide_kernel(
     /* B operands: chunk kb of a line, halves 0 and 1, of row p; chunk 4 + kb is eight 16-byte
      * units on (the swizzle moves the low three bits only) */
     const int x0 = 512 * p + 16 * ((2 * kb) ^ (p & 7)), x1 = x0 ^ 16;
-    const int ca = first ? kb : 4 + kb, cb = first ? 4 + kb : kb;
+    /* codes: a load's row and chunk of this lane, and their turn into operands */
+    const int lr = l >> 3, lc8 = l & 7;
+    uint8_t* const turn = lg_lds + 2 * 8192 * NTG + 8 * 2 * 256 + kLinesTurn * wave;
+    const int twr = 128 * lr + 16 * (lc8 ^ lr), trd = 128 * p + 16 * (kb ^ (p & 7));
 
     const int nb = (blocks - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
     auto row0 = [&](int bi) -> int64_t {              /* past the last block: rows past N */
@@ -114,13 +118,13 @@ void logits_wide_kernel(
         const __amdgpu_buffer_rsrc_t rc = r3d_rsrc(codes + (rows ? n0 : 0) * K, rows * K);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int ka = 256 * c.w + 128 * j + 16 * ca, kc = 256 * c.w + 128 * j + 16 * cb;
+            const int ka = 256 * c.w + 128 * j + 16 * lc8;
 #pragma unroll
             for (int t = 0; t < TW; ++t) {
                 cw[buf][t][2 * j] = r3d_buf_ld16_stream(
-                    rc, ka < K ? (uint32_t)((16 * t + r8) * K + ka) : kLgOob);
+                    rc, ka < K ? (uint32_t)((16 * t + lr) * K + ka) : kLgOob);
                 cw[buf][t][2 * j + 1] = r3d_buf_ld16_stream(
-                    rc, kc < K ? (uint32_t)((16 * t + 8 + r8) * K + kc) : kLgOob);
+                    rc, ka < K ? (uint32_t)((16 * t + 8 + lr) * K + ka) : kLgOob);
             }
         }
     };
@@ -137,7 +141,7 @@ void logits_wide_kernel(
             r3d_i32x4 v[TW][2];
 #pragma unroll
             for (int t = 0; t < TW; ++t)
-                r3d_lines_fix(cw[buf][t][2 * j], cw[buf][t][2 * j + 1], first, v[t][0], v[t][1]);
+                r3d_lines_turn(turn, twr, trd, cw[buf][t][2 * j], cw[buf][t][2 * j + 1], v[t][0], v[t][1]);
             r3d_f32x4 blk[TW][NTG];
 #pragma unroll
             for (int t = 0; t < TW; ++t)

@@ -396,7 +396,7 @@ LogitsGeom logits_geom(const LogitsPlan& P, int cus, int per_cu);
 /* The wide walk (r3d_logits_wide.h): its LDS at ntg activation groups (two windows of x, then
  * 8 waves' scale tables), its tiles a wave, and its grid (two workgroups a compute unit,
  * chunks counting blocks of 128 wtw head rows; passes of 64 activation rows). */
-constexpr int logits_wide_lds(int ntg) { return 2 * 8192 * ntg + 8 * 2 * 256; }
+constexpr int logits_wide_lds(int ntg) { return 2 * 8192 * ntg + 8 * 2 * 256 + 8 * kLinesTurn; }
 int logits_wide_tiles(int64_t N, int ntg, int cus);
 LogitsGeom logits_wide_geom(const LogitsPlan& P, int cus);
 
