@@ -142,11 +142,12 @@ static int launch_lines(const GemmPlan& P, const LinesGeom& g, hipStream_t strea
                         int passes = 1) {
     if (forced_fail(passes > 1 ? "skinny" : "lines"))
         return launch_failed(passes > 1 ? "skinny line GEMV" : "line decode GEMV", hipSuccess);
-    const dim3 grid((unsigned)g.blocks, (unsigned)passes), block((unsigned)(64 * g.wv));
+    const dim3 grid((unsigned)(g.blocks * passes)), block((unsigned)(64 * g.wv));
     const int64_t lim = (int64_t)1 << 31;
     int cl = 0;
     while (cl < 3 && (1 << cl) < g.chunks) ++cl;
-    if (P.M < 1 || P.M > 127 || g.chunks != 1 << cl || g.wv != (cl == 3 ? 8 : 4) ||
+    if (P.M < 1 || P.M > 16 * passes || passes > 4 || g.blocks * passes > 0x7FFFFFFF ||
+        g.chunks != 1 << cl || g.wv != (cl == 3 ? 8 : 4) ||
         (g.wv == 8 && g.tw != 1) ||
         P.a_pitch >= lim || P.as_pitch >= lim || P.b_pitch >= lim || P.bs_pitch >= lim ||
         g.wlds != lines_wlds(P.enc, g.tw, P.K, g.chunks))
@@ -203,22 +204,24 @@ static hipError_t wide_launch(const GemmPlan& P, const WideGeom& w, int kc, floa
     const int pk = wide_pack((int)P.M, P.rblk == 128, P.a_pitch == P.K, P.as_pitch == P.K / 128);
     const int cgkc = w.cg | (kc << 16);
     const dim3 grid((unsigned)(w.ntiles * kc)), block(512);
-#define R3D_WIDE(ENC_, D_, NTG_)                                                           \
-    hipLaunchKernelGGL((gemv_wide_kernel<ENC_, 2, D_, NTG_>), grid, block, (size_t)w.lds,    \
+#define R3D_WIDE(ENC_, D_, NTG_, TURN_)                                                    \
+    hipLaunchKernelGGL((gemv_wide_kernel<ENC_, 2, D_, NTG_, TURN_>), grid, block, (size_t)w.lds, \
                        stream, P.A, P.AS, P.B, P.BS, (int)P.N, (int)P.K, (int)P.b_pitch,     \
                        (int)P.bs_pitch, pk, cgkc, (int)P.a_pitch, (int)P.as_pitch, part)
-#define R3D_WIDE_N(ENC_, D_)                                                                \
+#define R3D_WIDE_N(ENC_, D_, TURN_)                                                         \
     switch (w.ntg) {                                                                        \
-        case 1: R3D_WIDE(ENC_, D_, 1); break;                                               \
-        case 2: R3D_WIDE(ENC_, D_, 2); break;                                               \
-        case 3: R3D_WIDE(ENC_, D_, 3); break;                                               \
-        default: R3D_WIDE(ENC_, D_, 4); break;                                              \
+        case 1: R3D_WIDE(ENC_, D_, 1, TURN_); break;                                        \
+        case 2: R3D_WIDE(ENC_, D_, 2, TURN_); break;                                        \
+        case 3: R3D_WIDE(ENC_, D_, 3, TURN_); break;                                        \
+        default: R3D_WIDE(ENC_, D_, 4, TURN_); break;                                       \
     }
     if (w.ntg < 1 || w.ntg > 4 || w.d != 1) return hipErrorInvalidValue;
     if (P.enc == ENC_MXFP4A8) {
-        R3D_WIDE_N(ENC_MXFP4A8, 1)
+        R3D_WIDE_N(ENC_MXFP4A8, 1, false)
+    } else if (w.turn) {
+        R3D_WIDE_N(ENC_FP8A8, 1, true)
     } else {
-        R3D_WIDE_N(ENC_FP8A8, 1)
+        R3D_WIDE_N(ENC_FP8A8, 1, false)
     }
 #undef R3D_WIDE_N
 #undef R3D_WIDE
@@ -404,7 +407,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
         S.M = 16;
         LinesGeom lg{};
         int rc = RAD_E_DEVICE;
-        if (lines_fits(S) && lines_geom(P.enc, 16, P.N, P.K, 0, &lg) && lg.mt == 16) {
+        if (lines_fits(S) && lines_geom(P.enc, 16, P.N, P.K, 0, &lg, passes) && lg.mt == 16) {
             rc = launch_lines(P, lg, stream, passes);       /* all passes in one launch */
         } else {
             rc = RAD_OK;

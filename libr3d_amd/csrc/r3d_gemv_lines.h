@@ -46,19 +46,6 @@
 
 namespace r3d {
 
-/* (lo, hi) operand registers from the two loads of a line pair (see the header); `first`
- * is true in lanes 0-7 of every 16-lane row. */
-__device__ __forceinline__ void r3d_lines_fix(const r3d_i32x4& a, const r3d_i32x4& b, bool first,
-                                              r3d_i32x4& lo, r3d_i32x4& hi) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        lo[i] = first ? a[i] : b[i];
-        /* every lane takes b from lane p ^ 8, then lanes 0-7 (banks 0-1) take a from it */
-        const int t = __builtin_amdgcn_mov_dpp(b[i], 0x128, 0xF, 0xF, false);   /* row_ror:8 */
-        hi[i] = __builtin_amdgcn_update_dpp(t, a[i], 0x128, 0xF, 0x3, false);
-    }
-}
-
 /* (lo, hi) operand registers of 16 rows from their two loads (lane l of load h: row 8 h + l / 8,
  * chunk l % 8), through 2 KB of the wave's own LDS: row r's chunk c sits at
  * 128 r + 16 (c ^ r % 8), so eight lanes writing a row and eight lanes reading one chunk of
@@ -106,10 +93,25 @@ __global__ __launch_bounds__(64 * WV) void gemv_lines_kernel(
     const int cl = (pk >> 7) & 7, chunks = 1 << cl;
     const bool rblk128 = (pk >> 10) & 1, as_dense = (pk >> 11) & 1;
     const int groups = K >> 7;
-    /* grid.y > 1 (the skinny band): workgroup row y computes activation rows
-     * [16 y, 16 y + 16) of a taller A -- the same arithmetic as a 16-row call (AS moves
-     * with it in the staging below) */
-    const int m0 = 16 * (int)blockIdx.y;
+    /* M > 16 (the skinny band): pass y computes activation rows [16 y, 16 y + 16) of a taller
+     * A -- the same arithmetic as a 16-row call (AS moves with it in the staging below).  The
+     * passes over a weight block are neighbours on one XCD (workgroups go round-robin over the
+     * 8), so all but the first find it in the L2; the tail that 8 does not divide is in order. */
+    const int passes = (M + 15) >> 4;
+    int bx = blockIdx.x, py = 0;
+    if (passes > 1) {
+        const int whole = ((int)gridDim.x / (8 * passes)) * 8 * passes;
+        if (bx < whole) {
+            const int q = bx >> 3;
+            py = q % passes;
+            bx = (q / passes) * 8 + (bx & 7);
+        } else {
+            const int q = bx - whole;
+            py = q % passes;
+            bx = whole / passes + q / passes;
+        }
+    }
+    const int m0 = 16 * py;
     {
         A += (int64_t)m0 * a_pitch;
         Y += m0 * y_pitch;
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(64 * WV) void gemv_lines_kernel(
     const int units = (groups + G - 1) / G;
     const int tpb = WV >> cl;                              /* row blocks per workgroup */
     const int ti = wave >> cl, c = wave & (chunks - 1);
-    const int64_t n0 = ((int64_t)blockIdx.x * tpb + ti) * RW;
+    const int64_t n0 = ((int64_t)bx * tpb + ti) * RW;
     const int u0 = (units * c) >> cl;                      /* units < 2^21: no overflow */
     const int ns = ((units * (c + 1)) >> cl) - u0;         /* >= 1: chunks <= units */
     const int gmax = G * ((units + chunks - 1) >> cl);
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(64 * WV) void gemv_lines_kernel(
         float y = 0.0f;
         for (int cc = 0; cc < chunks; ++cc)
             y += rf[(((b * chunks + cc) * TW + t) * 64 + 16 * (rr >> 2) + tk) * 4 + (rr & 3)];
-        const int64_t n = ((int64_t)blockIdx.x * tpb + b) * RW + r;
+        const int64_t n = ((int64_t)bx * tpb + b) * RW + r;
         if (tk < M && n < N) Y[(int64_t)tk * y_pitch + n] = r3d_bf16_rne(y);
     }
 }

@@ -16,8 +16,10 @@
  *   * each wave stages its own rows' weight scales (mxfp4a8: [RW rows][cg] E8M0 dwords;
  *     fp8a8: [cg][RW] 4-byte slots, bf16 in the low half) after them;
  *   * the weights stream in whole 128-byte lines straight into the MFMA operand registers,
- *     D lines ahead in a register ring, exactly as the line GEMV's (r3d_gemv_lines.h: two
- *     loads per 16 rows, rows 0-7 and 8-15, rebuilt by one select and two DPP rotates);
+ *     D lines ahead in a register ring: two loads per 16 rows, rows 0-7 and 8-15, eight lanes
+ *     a line and turned in LDS as the line GEMV's (TURN: e4m3 where the LDS holds it), or a row
+ *     a lane, lane p the chunk ca = kb (p < 8) or 4 + kb of row p % 8 and then cb = 4 + kb or
+ *     kb of row 8 + p % 8, rebuilt by one select and two DPP rotates (r3d_lines_fix);
  *   * per K group, one v_mfma_scale_f32_16x16x128_f8f6f4 per (weight tile, 16-row group of
  *     activations): the weights are source A, the activation rows source B (from LDS), the
  *     E8M0 weight scales ride the scale operand (mxfp4a8); the result is scaled by the
@@ -41,6 +43,19 @@
 
 namespace r3d {
 
+/* (lo, hi) operand registers from the two loads of a line pair that gave each lane its own row (see the header); `first`
+ * is true in lanes 0-7 of every 16-lane row. */
+__device__ __forceinline__ void r3d_lines_fix(const r3d_i32x4& a, const r3d_i32x4& b, bool first,
+                                              r3d_i32x4& lo, r3d_i32x4& hi) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lo[i] = first ? a[i] : b[i];
+        /* every lane takes b from lane p ^ 8, then lanes 0-7 (banks 0-1) take a from it */
+        const int t = __builtin_amdgcn_mov_dpp(b[i], 0x128, 0xF, 0xF, false);   /* row_ror:8 */
+        hi[i] = __builtin_amdgcn_update_dpp(t, a[i], 0x128, 0xF, 0x3, false);
+    }
+}
+
 template <int TW>
 struct WideUnit {
     r3d_i32x4 w0[TW], w1[TW];
@@ -59,7 +74,7 @@ constexpr int wide_pack(int M, bool rblk128, bool a_dense, bool as_dense) {
  * activation pitches follow them and are fetched only when the rows are not dense; part is
  * first used after the K walk.  Pitches in bytes (b, a), bf16 / E8M0 elements (bs) or
  * floats (as), all below 2^31. */
-template <int ENC, int TW, int D, int NTG>
+template <int ENC, int TW, int D, int NTG, bool TURN>
 __global__ __launch_bounds__(512) void gemv_wide_kernel(
     const uint8_t* A, const float* AS, const uint8_t* B, const void* BSv,
     int N, int K, int b_pitch, int bs_pitch, int pk, int cgkc,
@@ -165,12 +180,17 @@ __global__ __launch_bounds__(512) void gemv_wide_kernel(
     const int64_t rows = N - n0 < RW ? (N - n0 > 0 ? N - n0 : 0) : RW;   /* 0: an empty wave */
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(B + n0 * b_pitch), (short)0, (int)(rows * b_pitch), 0x00020000);
-    const int ca = p < 8 ? kb : 4 + kb, cb = p < 8 ? 4 + kb : kb;
+    /* TURN: a load's lanes walk whole lines, eight to a row, and 2 KB of LDS turns two loads into
+     * operands (r3d_gemv_lines.h); else each lane has its row and the two loads are shuffled */
+    const int lr = TURN ? lane >> 3 : r8;
+    const int ca = TURN ? lane & 7 : first ? kb : 4 + kb, cb = TURN ? ca : first ? 4 + kb : kb;
+    uint8_t* const turn = smem + sc_off + WV * sclds + kLinesTurn * wave;
+    const int twr = 128 * lr + 16 * (ca ^ lr), trd = 128 * p + 16 * (kb ^ (p & 7));
     uint32_t wa[TW], wb[TW];
 #pragma unroll
     for (int tt = 0; tt < TW; ++tt) {
-        wa[tt] = (uint32_t)((16 * tt + r8) * b_pitch + 16 * ca + 128 * (int64_t)u0);
-        wb[tt] = (uint32_t)((16 * tt + 8 + r8) * b_pitch + 16 * cb + 128 * (int64_t)u0);
+        wa[tt] = (uint32_t)((16 * tt + lr) * b_pitch + 16 * ca + 128 * (int64_t)u0);
+        wb[tt] = (uint32_t)((16 * tt + 8 + lr) * b_pitch + 16 * cb + 128 * (int64_t)u0);
     }
     using Unit = WideUnit<TW>;
     const uint32_t kSkip = 0x80000000u;
@@ -215,7 +235,10 @@ __global__ __launch_bounds__(512) void gemv_wide_kernel(
     auto consume = [&](const Unit& v, int s) {
         r3d_i32x4 wlo[TW], whi[TW];
 #pragma unroll
-        for (int tt = 0; tt < TW; ++tt) r3d_lines_fix(v.w0[tt], v.w1[tt], first, wlo[tt], whi[tt]);
+        for (int tt = 0; tt < TW; ++tt) {
+            if constexpr (TURN) r3d_lines_turn(turn, twr, trd, v.w0[tt], v.w1[tt], wlo[tt], whi[tt]);
+            else r3d_lines_fix(v.w0[tt], v.w1[tt], first, wlo[tt], whi[tt]);
+        }
 #pragma unroll
         for (int h = 0; h < G; ++h) {
             const int gl = G * s + h;                      /* group inside the chunk */

@@ -425,7 +425,8 @@ bool lines_fits(const GemmPlan& P) {
 /* Line geometry: tw tiles per wave (policy or R3D_GFX950_LTW), then split K until about
  * env_lines_waves() waves are in flight (keeping >= 4 lines per chunk), or until a wave's
  * scale tables fit the LDS budget. */
-bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, LinesGeom* g) {
+bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, LinesGeom* g,
+                int passes) {
     /* M <= 4 shapes the quad GEMV cannot stage run faster on the 16-row GEMV's 4-row
      * instantiation (measured on MI355X at K = 21504) */
     if (M < 5 || M > 16 || N < 1 || K < 128 || K % 128 != 0) return false;
@@ -447,10 +448,13 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
      * activation rows e2m1 loads half as many activation bytes and keeps one tile up to 2^26
      * weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4). */
     const int etw = env_lines_tw();
-    const bool small = g->tiles <= 256 ||
+    /* the skinny band's passes are that many more tiles over the same weights (M = 60 as four
+     * passes of 3328 x 6656, e4m3: one tile 21.0, two 18.9) */
+    const int64_t pt = g->tiles * passes, work = N * K * passes;
+    const bool small = pt <= 256 ||
                        (enc == ENC_MXFP4A8 && g->mt == 8
-                            ? N * K < ((int64_t)1 << 26)
-                            : N * K < ((int64_t)45 << 20) && (g->tiles <= 768 || K < 1920));
+                            ? work < ((int64_t)1 << 26)
+                            : work < ((int64_t)45 << 20) && (pt <= 768 || K < 1920));
     g->tw = etw == 1 || etw == 2 || etw == 4 ? etw : small ? 1 : 2;
     g->nblk = (g->tiles + g->tw - 1) / g->tw;
     auto wlds_of = [&](int c) { return lines_wlds(enc, g->tw, K, c); };
@@ -464,7 +468,7 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
          * has a CU to itself and two units a wave (4 -> 8: e4m3 2304 x 2560 5.0 -> 4.7,
          * 512 x 17152 14.2 -> 12.1; 16 chunks give no more). */
         c = g->units >= (g->tiles < 32 ? 9 : 4) ? 4 : g->units >= 2 ? 2 : 1;
-        if (g->units >= 16 && g->tiles <= 256) c = 8;
+        if (g->units >= 16 && pt <= 256) c = 8;
     } else {
         const int64_t target = env_lines_waves();
         while (c < 4 && g->units >= 8 * c &&
@@ -789,7 +793,12 @@ static bool wide_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t kc0, Wid
     if (lds > kWideMaxLds) return false;
     w->cg = (int)cg;
     w->sclds = (int)scl;
-    w->lds = (int)lds;
+    /* e4m3 loads whole lines and turns them in LDS where that fits (M = 17..64, us: 640 x 7424
+     * 10.6 -> 9.4, 13568 x 1408 14.0 -> 12.9, 11648 x 7552 24.9 -> 24.0); e2m1, with half the
+     * bytes per MFMA, gains up to M = 32 and loses past it (2703 x 1920 10.4 -> 10.2, but
+     * 9984 x 6272 at M = 55 17.5 -> 19.0) and keeps the shuffled loads. */
+    w->turn = enc == ENC_FP8A8 && lds + 8 * kLinesTurn <= kWideTurnLds;
+    w->lds = (int)lds + (w->turn ? 8 * kLinesTurn : 0);
     w->d = 1;
     return true;
 }

@@ -178,7 +178,8 @@ bool quad_fits(const GemmPlan& P);
  * 1/2/4 pin the split, anything else above 0 leaves the line kernel. */
 constexpr int kLinesMaxLds = 48 * 1024;     /* scale tables of 4 waves */
 constexpr int kLinesTurn = 2048;            /* a wave's LDS for turning loads into operands */
-bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, LinesGeom* g);
+bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, LinesGeom* g,
+                int passes = 1);
 /* The line kernel addresses a wave's (up to 64) weight rows and the whole activation plane through
  * buffer resources: both must span less than 2^31 bytes. */
 bool lines_fits(const GemmPlan& P);
@@ -223,9 +224,11 @@ int prefill_mx_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, Prefil
 struct WideGeom {
     int tw, d;
     int cg, ntg, sclds, lds;
+    bool turn;               /* weight lines loaded whole and turned in LDS */
     int64_t ntiles;
 };
 constexpr int kWideMaxLds = 152 * 1024;
+constexpr int kWideTurnLds = 160 * 1024;    /* with the 8 waves' turn buffers: a CU's LDS */
 
 /* Split K on the tile rows (mxfp4a8, fp8a8) up to M = 128, where a narrow N leaves most
  * CUs idle under the prefill pipeline's one tile per 128 weight rows: the K steps are cut

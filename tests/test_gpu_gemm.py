@@ -153,6 +153,29 @@ def test_decode_lines_split_rule(gpu, dtype, N, K, geom, M):
     _check(row, dtype, A, AS, B, BS, M, N, K, gpu)
 
 
+@pytest.mark.parametrize("dtype,M,N,K", [
+    # workgroups a multiple of 8 and not, fewer than 8, one and two tiles a wave, 4 and 8 chunks
+    ("fp8a8", 17, 100, 640), ("fp8a8", 33, 1040, 640), ("fp8a8", 64, 2048, 2048),
+    ("fp8a8", 50, 1000, 3200), ("mxfp4a8", 18, 130, 384), ("mxfp4a8", 47, 1300, 896),
+    ("mxfp4a8", 64, 500, 4224), ("fp8a8", 40, 6432, 5504)])
+def test_skinny_passes(gpu, dtype, M, N, K):
+    """No scratch: 16-row passes whose workgroups are interleaved over a weight block."""
+    A, AS, B, BS = (_mx_case(M, N, K, M + N + K) if dtype == "mxfp4a8"
+                    else _f8_case(M, N, K, M + N + K, 1))
+    _check(MX_TILE if dtype == "mxfp4a8" else F8_TILE, dtype, A, AS, B, BS, M, N, K, gpu)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 300, 4096), (64, 12288, 8192), (17, 640, 2176),
+                                   (48, 12300, 7808)])
+@pytest.mark.parametrize("rblk", [1, 128])
+def test_fp8_split_gemv_loads(gpu, M, N, K, rblk):
+    """The K-split GEMV where a workgroup's LDS holds the turn buffers and where it does not."""
+    if rblk == 128 and N % 128:
+        N += 128 - N % 128
+    A, AS, B, BS = _f8_case(M, N, K, M + N + K, rblk)
+    _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk, scratch="hook")
+
+
 @pytest.mark.parametrize("pad,offset", [(4, 0), (0, 4), (12, 8)])
 def test_mxfp4_decode_scale_plane_layouts(gpu, pad, offset):
     """The E8M0 plane as a padded-pitch and/or 4-byte (not 16-byte) aligned view: the decode
