@@ -23,6 +23,11 @@
 typedef int   r3d_i32x8 __attribute__((ext_vector_type(8)));
 typedef int   r3d_i32x4 __attribute__((ext_vector_type(4)));
 typedef float r3d_f32x4 __attribute__((ext_vector_type(4)));
+/* the same at element alignment: rows of a ragged pitch leave and arrive in 16-byte accesses too
+ * (gfx950 global memory takes them unaligned) */
+typedef int   r3d_i32x4_u2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float r3d_f32x4_u4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t r3d_u32x2_u2 __attribute__((ext_vector_type(2), aligned(2)));
 
 enum { R3D_MFMA_FP8 = 0, R3D_MFMA_FP4 = 4 };
 enum { R3D_E8M0_ONE = 127 };

@@ -318,7 +318,6 @@ __global__ __launch_bounds__(512) void gemv_wide_kernel(
     /* ---- 4. the partial tile: lane l holds rows 4 (l / 16) + i of each weight tile for
      * activation row 16 tg + l % 16 -- four consecutive columns of plane c */
     float* pp = part + (int64_t)c * M * N;
-    const bool v4 = (N & 3) == 0;
 #pragma unroll
     for (int tt = 0; tt < TW; ++tt)
 #pragma unroll
@@ -328,8 +327,8 @@ __global__ __launch_bounds__(512) void gemv_wide_kernel(
             if (m >= M || n >= N) continue;
             float* d = pp + (int64_t)m * N + n;
             const r3d_f32x4 v = acc[tt][tg];
-            if (v4) {
-                *reinterpret_cast<r3d_f32x4*>(d) = v;
+            if (n + 4 <= N) {
+                *reinterpret_cast<r3d_f32x4_u4*>(d) = v;
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)

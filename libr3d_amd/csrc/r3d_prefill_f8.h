@@ -316,7 +316,6 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
     uint16_t* const Y = P.Y;
     if (P.part) {
         float* const pp = P.part;
-        const bool v4 = (N & 3) == 0;
 #pragma unroll
         for (int ni = 0; ni < WNF; ++ni)
 #pragma unroll
@@ -326,8 +325,8 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
                 if (m >= M || n >= N) continue;
                 const r3d_f32x4 v = acc[ni][mi];
                 float* o = pp + m * N + n;
-                if (v4) {
-                    *reinterpret_cast<r3d_f32x4*>(o) = v;
+                if (n + 4 <= N) {
+                    *reinterpret_cast<r3d_f32x4_u4*>(o) = v;
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -348,15 +347,14 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
                 make_uint2(r3d_pack_bf16x2(v[0], v[1]), r3d_pack_bf16x2(v[2], v[3]));
         }
     __syncthreads();
-    const bool vec = ((uintptr_t)Y & 15) == 0 && (y_pitch & 7) == 0;
     for (int e = threadIdx.x; e < L::BM * CPR; e += 512) {
         const int r = e / CPR, c = e - (e / CPR) * CPR;
         const int64_t m = m0 + r, n = n0 + 8 * c;
         if (m >= M || n >= N) continue;
         const r3d_i32x4 v = *reinterpret_cast<const r3d_i32x4*>(smem + r * YP + 16 * c);
         uint16_t* yp = Y + m * y_pitch + n;
-        if (vec && n + 8 <= N) {
-            *reinterpret_cast<r3d_i32x4*>(yp) = v;
+        if (n + 8 <= N) {
+            *reinterpret_cast<r3d_i32x4_u2*>(yp) = v;
         } else {
             const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
             for (int i = 0; i < 8; ++i)

@@ -176,6 +176,19 @@ def test_fp8_split_gemv_loads(gpu, M, N, K, rblk):
     _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk, scratch="hook")
 
 
+@pytest.mark.parametrize("N", [257, 258, 259, 261, 262, 263])
+@pytest.mark.parametrize("M,scratch", [(20, "hook"), (100, "hook"), (100, None), (300, "hook"),
+                                       (300, None)])
+def test_ragged_row_stores(gpu, M, N, scratch):
+    """Every remainder of N by 4 and 8: partial planes, their sum and the bf16 rows are 16-byte
+    accesses at element alignment, with a column tail by the element."""
+    K = 2048
+    A, AS, B, BS = _mx_case(M, N, K, M + N)
+    _check(MX_TILE, "mxfp4a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
+    A, AS, B, BS = _f8_case(M, N, K, M + N, 1)
+    _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
+
+
 @pytest.mark.parametrize("pad,offset", [(4, 0), (0, 4), (12, 8)])
 def test_mxfp4_decode_scale_plane_layouts(gpu, pad, offset):
     """The E8M0 plane as a padded-pitch and/or 4-byte (not 16-byte) aligned view: the decode
