@@ -50,9 +50,10 @@ int r3d_rad_gemm_nt_q_fp8(const RadArgs* a, RadStream s);
 
 /* Scratch hooks (RadKernelInfo::scratch) of the two tile rows, r3d_rad_gemm_nt_q (mxfp4a8)
  * and r3d_rad_gemm_nt_q_fp8.  No counterpart in the reference, whose tile rows take no
- * scratch: up to M = 128 on an N too narrow to fill the chip with 128-row tiles, these rows
- * split K across workgroups into f32 partial planes in RadArgs::scratch and sum them in
- * order on the same stream.  The hook returns the bytes of those planes (kc * M * N * 4 at
+ * scratch: up to M = 128 on an N too narrow to fill the chip with 128-row tiles, and from
+ * M = 144 on where a whole-K walk of the larger tiles would leave compute units idle (planes of
+ * at most 256 MiB), these rows split K across workgroups into f32 partial planes in
+ * RadArgs::scratch and sum them in order on the same stream.  The hook returns the bytes of those planes (kc * M * N * 4 at
  * the N and K parameters and M = numel(y) / N -- without y the M parameter, else 128), 0 when no split applies.
  * The scratch is optional: a launch without it, or with less, or at an address that is not
  * 16-byte aligned, runs the unsplit arms (never a refusal). */
@@ -86,7 +87,9 @@ int64_t r3d_rad_gemm_nt_q_fp8_decode_scratch(const RadArgs* a);
 int r3d_rad_gemm_nt_q_mxfp4a16(const RadArgs* a, RadStream s);
 
 /* The mxfp4a16 row's scratch hook (RadKernelInfo::scratch): bytes of launch scratch for
- * the M and K parameters, 0 when either is missing.  Same role as the reference's
+ * the M and K parameters, 0 when either is missing: the quantised activations, and after them
+ * the f32 partial planes of a K split where one pays (from M = 144 on, with the N parameter).
+ * A launch needs the former; with less than both it runs unsplit.  Same role as the reference's
  * src/r3d_gemm_fp8a8.hip:1249-1253. */
 int64_t r3d_rad_gemm_nt_q_mxfp4a16_scratch(const RadArgs* a);
 

@@ -444,9 +444,9 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
      * 5.6 7.1, 8192 x 5376 8.1 8.3, 5120 x 10624 13.9 13.2, 21504 x 5376 19.1 17.6; e4m3
      * 2304 x 5376 7.0 9.1, 5120 x 10624 16.4 15.5, 21504 x 5376 24.2 21.6.  Past 768 tiles the
      * waves of one tile no longer fit the chip at once, unless K is short (e2m1 16384 x 2560 9.7
-     * 8.0, 15104 x 1920 8.7 7.2, 21504 x 1536 7.6 8.7); up to 256 tiles the split in 8 below needs one.  With 8
-     * activation rows e2m1 loads half as many activation bytes and keeps one tile up to 2^26
-     * weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4). */
+     * 8.0, 15104 x 1920 8.7 7.2, 21504 x 1536 7.6 8.7); up to 256 tiles the split in 8 below needs
+     * one.  With 8 activation rows e2m1 loads half as many activation bytes and keeps one tile
+     * up to 2^26 weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4). */
     const int etw = env_lines_tw();
     /* the skinny band's passes are that many more tiles over the same weights (M = 60 as four
      * passes of 3328 x 6656, e4m3: one tile 21.0, two 18.9) */
@@ -805,7 +805,12 @@ static bool wide_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t kc0, Wid
 
 int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int* cst,
                 PrefillGeom* g, WideGeom* w) {
+    static const long long lever = [] {
+        const char* e = getenv("R3D_GFX950_SPLITK_UNITS");
+        return e ? atoll(e) : -1LL;
+    }();
     if (M > 128 && N > 0 && K >= 128) {
+        if (lever == 0) return 0;
         int c = 0;
         const bool f8 = enc == ENC_FP8A8;
         const int k = f8 ? prefill_f8_splitk(M, N, K, ncu, &c, g) : prefill_mx_splitk(M, N, K, ncu, &c, g);
@@ -828,10 +833,6 @@ int splitk_plan(int enc, int64_t M, int64_t N, int64_t K, int ncu, int* kc, int*
         if (cst) *cst = c;
         return 2;
     }
-    static const long long lever = [] {
-        const char* e = getenv("R3D_GFX950_SPLITK_UNITS");
-        return e ? atoll(e) : -1LL;
-    }();
     if (ncu <= 0) ncu = 256;
     const int64_t target = lever >= 0 ? lever : ncu;
     /* units aim at the target over the GEMV's 256-row tiles, at least kSplitMinSteps groups a

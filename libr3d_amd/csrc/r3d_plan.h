@@ -253,7 +253,8 @@ int64_t tile_splitk_bytes(int enc, int64_t M, int64_t N, int64_t K, int ncu);
 int64_t mxfp4a16_split_offset(int64_t M, int64_t K);
 int64_t mxfp4a16_hook_bytes(int64_t M, int64_t N, int64_t K, int ncu);
 /* The tile rows' scratch hook: tile_splitk_bytes at the args' N and K and M (numel(y) / N,
- * else the "M" param, else 128 -- the largest M the split takes); 0 without N or K. */
+ * else the "M" param, else 128 -- past it a call without either gets no planes); 0 without N
+ * or K. */
 int64_t tile_scratch_bytes(const RadArgs* a, int enc, int ncu);
 
 /* The decode rows' K split over launch scratch: the skinny-band GEMV's split (splitk_plan

@@ -135,7 +135,8 @@ def test_plan_wide_walk():
         assert rc == R.RAD_OK and g["walk"] == walk, (M, N, g)
         assert (g["mt"], g["passes"]) == (str(mt), str(passes)), (M, N, g)
         if walk.startswith("wide"):
-            assert g["lds"] == str(1024 * mt + 4096), g
+            # two windows of activation rows, the scale tables, 2 KB a wave to turn the codes in
+            assert g["lds"] == str(1024 * mt + 4096 + 8 * 2048), g
     ops, keep = _ops(M=16, N=16384, K=260)
     assert _desc(ops)[1]["walk"] == "dword"
 
