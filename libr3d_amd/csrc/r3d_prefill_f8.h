@@ -56,8 +56,8 @@ struct F8Args {
     float* part;                     /* this unit's f32 plane, or null: the whole walk into Y */
 };
 
-/* One tile at (n0, m0) over the groups [s0, s0 + steps).  F8_CHAN: false, and nothing done,
- * where some row's scale is not one finite value over them. */
+/* One tile at (n0, m0) over the groups [s0, s0 + steps).  F8_CHAN: false, and nothing written,
+ * where some row's scale is not one finite value over them or a result is not finite. */
 template <int WMW, int SC>
 __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, int64_t n0,
                                                 int64_t m0, int s0, int steps) {
@@ -302,6 +302,11 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
 #pragma unroll
         for (int mi = 0; mi < WMW; ++mi) asm volatile("" : "+v"(acc[ni][mi]));
     if (SC == F8_CHAN) {
+        /* sum(D * sa) leaves the f32 range before sum((D * sa) * sb) does where sb < 1, and a sum
+         * that left it stays Inf or NaN: a tile with such a result takes the per-group walk.  The
+         * largest magnitude, NaN above all, in half an instruction an element
+         * (300 x 2050 x 8192 split 30.1 -> 30.6 us, 512 x 5376 x 21504 94.0 -> 94.8). */
+        float big = 0.0f;
 #pragma unroll
         for (int ni = 0; ni < WNF; ++ni)
 #pragma unroll
@@ -310,7 +315,18 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
                 const float sb = __uint_as_float((uint32_t)BS[(n < N ? n : N - 1) * bs_pitch + s0] << 16);
 #pragma unroll
                 for (int mi = 0; mi < WMW; ++mi) acc[ni][mi][i] *= sb;
+#pragma unroll
+                for (int mi = 0; mi < WMW; mi += 2)
+                    big = __builtin_elementwise_maximum(
+                        __builtin_elementwise_maximum(fabsf(acc[ni][mi][i]), fabsf(acc[ni][mi + 1][i])), big);
             }
+        const uint32_t fin = __all(big < __builtin_inff());
+        if (lane == 0) flag[wave] = fin;
+        __syncthreads();
+        uint32_t f = 1;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f &= flag[i];
+        if (__builtin_amdgcn_readfirstlane(f) == 0) return false;
     }
 
     uint16_t* const Y = P.Y;

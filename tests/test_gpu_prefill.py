@@ -203,6 +203,24 @@ def test_fp8_wide_tile_non_finite_row_scale(gpu, bad):
     assert c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0 and c["max_viol"] <= 1.0, c
 
 
+@pytest.mark.parametrize("M,N,K,scratch", [(300, 21700, 384, None), (1030, 8448, 256, None),
+                                           (260, 514, 5376, "hook")])
+def test_fp8_wide_tile_large_token_scale(gpu, M, N, K, scratch):
+    """One scale a row, a token scale of 1e31 on codes of 448: every group's D * sa is finite
+    (2.6e38) and any two overflow, but the rows' 1e-10 scales bring the per-group products to
+    2.6e28.  The result is the per-group order's: finite, within the bound."""
+    from tests.test_gpu_gemm import F8_TILE, _check, _f8_case
+    A, AS, B, BS = _f8_case(M, N, K, M + K, 1)
+    BS = np.repeat(BS[:, :1], K // 128, axis=1).copy()
+    for m in (7, M - 1):
+        A[m], AS[m] = 0x7E, 1e31
+    for n in (3, 300, N - 1):
+        B[n], BS[n] = 0x7E, synth.bf16_bits(np.array([1e-10], np.float32))[0]
+    assert _wide_route(M, N, K, 1, scratch)
+    _, Y = _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
+    assert np.isfinite(O.bf16_to_f32(Y)[:, [3, 300, N - 1]]).all()
+
+
 MX_SPLIT = [(144, 300, 8192), (260, 514, 5376), (513, 130, 6144)]   # M, N, K
 
 
