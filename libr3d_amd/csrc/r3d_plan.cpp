@@ -446,15 +446,19 @@ bool lines_geom(int enc, int64_t M, int64_t N, int64_t K, int64_t force_chunks, 
      * waves of one tile no longer fit the chip at once, unless K is short (e2m1 16384 x 2560 9.7
      * 8.0, 15104 x 1920 8.7 7.2, 21504 x 1536 7.6 8.7); up to 256 tiles the split in 8 below needs
      * one.  With 8 activation rows e2m1 loads half as many activation bytes and keeps one tile
-     * up to 2^26 weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4). */
+     * up to 2^26 weights (5120 x 10624 at M = 6 11.4 11.8, 16384 x 2560 6.9 7.4); with 9 or 10 the
+     * second load of a group finds one or two distinct rows, and up to 384 tiles one tile stays
+     * the faster one to 57 M (4608 x 10624 at M = 9 13.3 14.2, 5120 x 10624 13.6 14.5,
+     * 4352 x 12800 13.8 14.4; at M = 13 14.9 15.2 and 15.0 14.7 at the latter two). */
     const int etw = env_lines_tw();
     /* the skinny band's passes are that many more tiles over the same weights (M = 60 as four
      * passes of 3328 x 6656, e4m3: one tile 21.0, two 18.9) */
     const int64_t pt = g->tiles * passes, work = N * K * passes;
+    const bool few = enc == ENC_MXFP4A8 && M <= 10 && pt <= 384;
     const bool small = pt <= 256 ||
                        (enc == ENC_MXFP4A8 && g->mt == 8
                             ? work < ((int64_t)1 << 26)
-                            : work < ((int64_t)45 << 20) && (pt <= 768 || K < 1920));
+                            : work < ((int64_t)(few ? 57 : 45) << 20) && (pt <= 768 || K < 1920));
     g->tw = etw == 1 || etw == 2 || etw == 4 ? etw : small ? 1 : 2;
     g->nblk = (g->tiles + g->tw - 1) / g->tw;
     auto wlds_of = [&](int c) { return lines_wlds(enc, g->tw, K, c); };

@@ -336,6 +336,18 @@ def test_tile_splitk_hook_and_arm():
         assert R.row_scratch_bytes("gemm_nt_q_mxfp4", ops) == (6 if M > 64 else 12) * M * 5376 * 4
 
 
+@pytest.mark.parametrize("M,N,K,tw", [
+    # 9 and 10 rows keep one tile a wave up to 57 M weights and 384 tiles; 11 and more to 45 M
+    (9, 4608, 10624, 1), (10, 5120, 10624, 1), (10, 6144, 9600, 1), (10, 6144, 9728, 2),
+    (10, 6160, 8192, 2), (11, 4608, 10624, 2), (16, 4608, 10112, 1), (16, 4608, 10240, 2),
+    # 5 to 8 rows to 2^26
+    (8, 6144, 10880, 1)])
+def test_lines_tiles_rule(M, N, K, tw):
+    ops, keep = _mx_ops(M=M, N=N, K=K)
+    g = _geom(R.describe("gemm_nt_q_mxfp4_decode", ops)[1])
+    assert (g["kernel"], g["tw"]) == ("lines", str(tw)), g
+
+
 def test_decode_split_hook_and_arm():
     """The decode rows' scratch hook sizes the skinny-band GEMV's K split (kc * M * N * 4)
     where the quad GEMV does not take the launch and the plane holds at least 2^26 weights,
