@@ -1284,7 +1284,7 @@ int plan_logits_e4m3(const RadArgs* a, const RadPlanesHead* hh, LogitsPlan* P, b
      * offsets are 32-bit. */
     if (!P->ua && M > 8 && N >= 128 * 128 && 2 * 64 * x_pitch < 0x7FFFFFFFLL) {
         P->wide = (int)(M >= 64 ? 4 : (M + 15) / 16);
-        P->wtw = logits_wide_tiles(N, P->wide, cu_count());
+        P->wtw = logits_wide_tiles(N, K, P->wide, cu_count());
         P->lds = logits_wide_lds(P->wide);
     }
     LogitsGuard& g = P->guard;
@@ -1307,17 +1307,21 @@ LogitsGeom logits_geom(const LogitsPlan& P, int cus, int per_cu) {
     return g;
 }
 
-/* Tiles a wave of the wide walk.  Two halve the restaging of the activation rows; one deals
- * the head over the 2 x cus workgroups in blocks half the size.  A round of one-tile blocks
- * costs a half of a two-tile round and f more (262144 x 5376, 4 rounds against 2 x 2: 1.07 at
- * 16 activation rows, 1.13 at 32, 1.23 at 64), so one tile runs where its rounds cost less:
- * 151936 x 4096 (3 rounds against 2 x 2) M = 16 132 against 146 us, M = 32 144 against 156,
- * but M = 64 183 against 175; 32000 x 4096 (1 against 2 x 1) 31 against 42 and, at 64, 41
- * against 52. */
-int logits_wide_tiles(int64_t N, int ntg, int cus) {
-    const int64_t wgs = 2 * (int64_t)(cus > 0 ? cus : 256);
-    const int64_t r1 = ((N + 127) / 128 + wgs - 1) / wgs, r2 = ((N + 255) / 256 + wgs - 1) / wgs;
-    return r1 * (ntg <= 2 ? 115 : 140) < 2 * r2 * 100 ? 1 : 2;
+/* Tiles a wave of the wide walk.  Two halve the restaging of the activation rows and one deals
+ * the head in blocks half the size.  A compute unit's registers hold two workgroups of one tile
+ * up to 32 activation rows (ntg 2), one otherwise, so a round -- a block a slot -- is 256 head
+ * rows a CU either way up to ntg 2, and one tile also fills half a round in half the time: it
+ * runs where N leaves the last round at most half full (us at K = 5120, M = 16, one tile and two:
+ * 98304 88 102, 151936 141 149; but 65536 60 57, 262144 231 215).  Past ntg 2 a round of one tile
+ * is 128 rows a CU and takes 1 / 1.5 of one of two (M = 64, K = 5376: 32000 55 74, 65536 111 86,
+ * 98304 156 149, 262144 393 328).  At K a multiple of 4096 the 32 rows of two tiles start on one
+ * memory channel, and one tile runs wherever it fills the chip as well (M = 16, K = 4096: 262144
+ * 197 232, 128256 102 119, 65536 58 63; K = 8192: 128256 196 225, 65536 100 103). */
+int logits_wide_tiles(int64_t N, int64_t K, int ntg, int cus) {
+    const int64_t rows = 128 * (int64_t)(cus > 0 ? cus : 256);
+    const int64_t h1 = (N + rows - 1) / rows, r2 = (N + 2 * rows - 1) / (2 * rows);
+    if (ntg > 2) return 100 * h1 < 150 * r2 ? 1 : 2;
+    return K % 4096 == 0 || 104 * h1 < 200 * r2 ? 1 : 2;
 }
 
 LogitsGeom logits_wide_geom(const LogitsPlan& P, int cus) {

@@ -398,10 +398,12 @@ struct LogitsGeom {
 };
 LogitsGeom logits_geom(const LogitsPlan& P, int cus, int per_cu);
 /* The wide walk (r3d_logits_wide.h): its LDS at ntg activation groups (two windows of x, then
- * 8 waves' scale tables), its tiles a wave, and its grid (two workgroups a compute unit,
- * chunks counting blocks of 128 wtw head rows; passes of 64 activation rows). */
+ * 8 waves' scale tables and turn buffers), its tiles a wave, and its grid: two workgroups a
+ * compute unit, which its registers hold at once at one tile and ntg <= 2; the others (156 to 252
+ * registers, and 84 KB of LDS at ntg 4) run one after the other.  chunks counts blocks of
+ * 128 wtw head rows; passes are of 64 activation rows. */
 constexpr int logits_wide_lds(int ntg) { return 2 * 8192 * ntg + 8 * 2 * 256 + 8 * kLinesTurn; }
-int logits_wide_tiles(int64_t N, int ntg, int cus);
+int logits_wide_tiles(int64_t N, int64_t K, int ntg, int cus);
 LogitsGeom logits_wide_geom(const LogitsPlan& P, int cus);
 
 /* The current device: gfx950 or not (answered once per device), and its compute units. */

@@ -124,7 +124,7 @@ def test_plan_geometry():
 
 def test_plan_wide_walk():
     """Past 8 activation rows a head of 16384 rows up takes the wide walk: 64 rows a pass, two
-    tiles a wave unless one-tile blocks' rounds over the 512 workgroups cost less.  8 rows, a
+    tiles a wave unless one-tile blocks fill the chip's rounds better.  8 rows, a
     small head, or operands off the vector walk's alignment keep the 4-row walk."""
     for M, N, walk, mt, passes in [(9, 262144, "wide2", 16, 1), (16, 151936, "wide1", 16, 1),
                                    (64, 151936, "wide2", 64, 1), (33, 32000, "wide1", 48, 1),
@@ -139,6 +139,21 @@ def test_plan_wide_walk():
             assert g["lds"] == str(1024 * mt + 4096 + 8 * 2048), g
     ops, keep = _ops(M=16, N=16384, K=260)
     assert _desc(ops)[1]["walk"] == "dword"
+
+
+@pytest.mark.parametrize("M,N,K,walk", [
+    # up to 32 rows a round is 65536 head rows at one tile and at two: one where the last round
+    # is at most half full, and wherever K is a multiple of 4096
+    (16, 32768, 1024, "wide1"), (16, 32769, 1024, "wide2"), (16, 65536, 1024, "wide2"),
+    (32, 98304, 5376, "wide1"), (32, 98305, 5376, "wide2"), (9, 65536, 4096, "wide1"),
+    (32, 262144, 4096, "wide1"),
+    # past it 32768 and 65536 rows, the former in two thirds of the time
+    (33, 32768, 1024, "wide1"), (64, 32769, 1024, "wide2"), (64, 65536, 5376, "wide2"),
+    (40, 98304, 1024, "wide2"), (40, 65536, 4096, "wide2")])
+def test_plan_wide_tiles(M, N, K, walk):
+    ops, keep = _ops(M=M, N=N, K=K)
+    rc, g = _desc(ops)
+    assert rc == R.RAD_OK and g["walk"] == walk, g
 
 
 def _hdr(N=1000, K=5376, sdt="bf16", br=1, **fields):
