@@ -552,7 +552,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
     if (const int w = mode == PF_F8 ? prefill_f8_wide(P.M, P.N, P.K, P.rblk, cu_count()) : 0) {
         const hipError_t e = launch_f8_wide(P, w, 1, (int)(P.K / 128), nullptr, stream);
         if (e == hipSuccess) {
-            debug_once("fp8a8 prefill, wide tile", 180 + w);
+            debug_once("fp8a8 prefill, wide tile", 184 + w / 2);   /* 184: four waves */
             return RAD_OK;
         }
         launch_failed("wide-tile prefill", e);

@@ -103,3 +103,14 @@ def test_split_kernel_lever(gpu, env, cases, kernel):
     for row, M, rc, guards, viol, unwritten, nan_mm in json.loads(line[7:]):
         assert rc == 0 and guards, (row, M, rc)
         assert viol <= 1.0 and unwritten == 0 and nan_mm == 0, (row, M, viol, unwritten)
+
+
+def test_debug_lines_of_both_fp8_tiles(gpu):
+    """R3D_DEBUG_GEMM names each arm once: the 256 x 128 wide tile's line must not use up the
+    four-wave tile's."""
+    cases = [("gemm_nt_q_fp8a8", "fp8a8", 300, 21504, 384), ("gemm_nt_q_fp8a8", "fp8a8", 130, 16896, 3072)]
+    p = subprocess.run([sys.executable, "-c", _CHILD % (ROOT, cases)], capture_output=True, text=True,
+                       env=dict(os.environ, R3D_DEBUG_GEMM="1"), timeout=300)
+    assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
+    for line in ("fp8a8 prefill, wide tile", "fp8a8 prefill, 128 x 256 on four waves"):
+        assert line + " launched" in p.stderr, p.stderr[-2000:]
