@@ -633,6 +633,22 @@ int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu) {
     return c8 <= c4 ? (c8 < base ? 8 : 0) : c4 < base ? 4 : 0;
 }
 
+PrefillGeom prefill_f8_geom(int wmw, int64_t M, int64_t N, int64_t K) {
+    PrefillGeom g{};
+    g.wnf = 4;
+    g.wmf = wmw;
+    g.nst = 2;
+    g.wv = 8;
+    g.bn = 256;
+    g.bm = 32 * wmw;
+    g.grid_n = (N + 255) / 256;
+    g.grid_m = (M + g.bm - 1) / g.bm;
+    g.tiles = g.grid_n * g.grid_m;
+    g.steps = (int)(K / 128);
+    g.lds = wmw == 8 ? PrefillF8Layout<8>::LDS_ALL : PrefillF8Layout<4>::LDS_ALL;
+    return g;
+}
+
 int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, PrefillGeom* g) {
     if (M < kPrefillSplitM || f8_tile_lever()) return 0;
     if (ncu <= 0) ncu = 256;
@@ -659,20 +675,7 @@ int prefill_f8_splitk(int64_t M, int64_t N, int64_t K, int ncu, int* cst, Prefil
     }
     if (!kbest) return 0;
     if (cst) *cst = (int)((steps + kbest - 1) / kbest);
-    if (g) {
-        *g = PrefillGeom{};
-        g->wnf = 4;
-        g->wmf = wbest;
-        g->nst = 2;
-        g->wv = 8;
-        g->bn = 256;
-        g->bm = 32 * wbest;
-        g->grid_n = (N + 255) / 256;
-        g->grid_m = (M + g->bm - 1) / g->bm;
-        g->tiles = g->grid_n * g->grid_m;
-        g->steps = (int)steps;
-        g->lds = wbest == 8 ? PrefillF8Layout<8>::LDS_ALL : PrefillF8Layout<4>::LDS_ALL;
-    }
+    if (g) *g = prefill_f8_geom(wbest, M, N, K);
     return (int)kbest;
 }
 
@@ -1590,6 +1593,7 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
         PrefillGeom g{};
         prefill_geom(P.M, P.N, P.K, mode, 256, &g);
         const int fw = mode == PF_F8 ? prefill_f8_wide(P.M, P.N, P.K, P.rblk, 256) : 0;
+        if (fw) g = prefill_f8_geom(fw, P.M, P.N, P.K);
         snprintf(buf, (size_t)len,
                  "arm=prefill enc=%s M=%lld N=%lld K=%lld bn=%d bm=%d waves=%d grid=%lldx%lld "
                  "tiles=%lld nst=%d lds=%d steps=%d rblk=%d nsplit=%lld quant=%s%s",
@@ -1598,7 +1602,6 @@ int describe(const char* row, const RadArgs* a, char* buf, int len) {
                  g.steps, P.rblk,
                  (long long)(mode == PF_F8 && g.wv == 4 ? prefill_f8_split_n(P.M, P.N, 256) : 0),
                  !a16 ? "none" : (P.ua & UA_QUANT) ? "elementwise" : "vector",
-                 /* the tile that takes the launch, ahead of the ones above */
                  fw == 8 ? " wide=256x256" : fw == 4 ? " wide=256x128" : "");
     }
     return RAD_OK;

@@ -208,6 +208,8 @@ int64_t prefill_f8_split_n(int64_t M, int64_t N, int ncu);
  * (8: 256 x 256, 4: 256 x 128) past 128 tokens where its rounds cost less than the tiles of
  * prefill_geom, else 0 (R3D_GFX950_F8_TILE keeps those).  rblk: the weight scale grid. */
 int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu);
+/* That tile's launch: wmw token fragments a wave. */
+PrefillGeom prefill_f8_geom(int wmw, int64_t M, int64_t N, int64_t K);
 /* The same tile with K split over launch scratch, from kPrefillSplitM tokens: kc, or 0; *cst
  * groups a chunk, *g the tile. */
 constexpr int64_t kPrefillSplitM = 144;

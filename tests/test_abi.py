@@ -653,7 +653,7 @@ def test_prefill_tile_choice_fills_the_last_round():
     assert (g["arm"], g["bn"], g["bm"], g["tiles"], g["steps"]) == ("prefill", "224", "256", "768", "42")
     assert int(g["lds"]) <= 160 * 1024
     # the f32-a_scale mode takes the same tile at config 3, 128-token tiles up to 128
-    # tokens; e4m3 weights run 128 x 256 on four waves past 128 tokens, 128 x 128 up to it
+    # tokens; e4m3 weights run 256 x 256 there, 128 x 128 up to 128 tokens
     ops, _ = _mx_ops(M=2048, N=21504, K=5376)
     g = _geom(R.describe("gemm_nt_q_mxfp4", ops)[1])
     assert (g["bn"], g["bm"], g["tiles"]) == ("224", "256", "768")
@@ -662,8 +662,8 @@ def test_prefill_tile_choice_fills_the_last_round():
     assert (g["bn"], g["bm"]) == ("128", "128")
     ops, _ = _f8_ops(M=2048, N=21504, K=5376)
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
-    assert (g["arm"], g["bn"], g["bm"], g["waves"], g["tiles"]) == ("prefill", "128", "256", "4", "1344")
-    assert int(g["lds"]) <= 160 * 1024
+    assert (g["arm"], g["bn"], g["bm"], g["waves"], g["tiles"]) == ("prefill", "256", "256", "8", "672")
+    assert (g["wide"], g["nsplit"]) == ("256x256", "0") and int(g["lds"]) <= 160 * 1024
     ops, _ = _f8_ops(M=128, N=21504, K=5376)
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
     assert (g["arm"], g["bn"], g["bm"], g["waves"]) == ("prefill", "128", "128", "8")
@@ -671,24 +671,31 @@ def test_prefill_tile_choice_fills_the_last_round():
     # at M = 256, N = 4096
     ops, _ = _f8_ops(M=256, N=4096, K=1024)
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
-    assert (g["bn"], g["bm"], g["waves"]) == ("128", "128", "8")
+    assert (g["bn"], g["bm"], g["waves"]) == ("128", "128", "8") and "wide" not in g
     # at M = 512, N = 21504: 3 rounds of 128 x 128, against one round of 128 x 256 over the
     # first 16384 weight rows and one of 128 x 128 over the rest (1.71 + 1)
     ops, _ = _f8_ops(M=512, N=21504, K=5376)
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
     assert (g["bn"], g["bm"], g["waves"], g["nsplit"]) == ("128", "256", "4", "16384")
-    # config 3's 1344 four-wave tiles are 5.25 rounds: the first 20480 weight rows run as 5
-    # whole rounds, the last 1024 as one launch of 128 x 128 tiles (5 x 1.71 + 1 < 6 x 1.71)
-    ops, _ = _f8_ops(M=2048, N=21504, K=5376)
-    assert _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])["nsplit"] == "20480"
-    # the remainder launch can make the four-wave tile pay where it alone would not:
-    # 260 tiles at M = 512, N = 16640 are 1 round + 4 tiles
-    ops, _ = _f8_ops(M=512, N=16640, K=1024)
+    assert int(g["lds"]) <= 160 * 1024
+    # M = 1200, N = 6656: 5 token tiles of 256 by 51 weight tiles are one round, the last weight
+    # tile is a launch of 128 x 128 tiles (1.71 + 1 < 2 x 1.71)
+    ops, _ = _f8_ops(M=1200, N=6656, K=1536)
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
-    assert (g["waves"], g["nsplit"]) == ("4", "16384"), g
-    ops, _ = _f8_ops(M=512, N=16384, K=1024)                  # 256 tiles: one whole round
+    assert (g["waves"], g["nsplit"]) == ("4", "6528"), g
+    # the remainder launch can make the four-wave tile pay where it alone would not:
+    # 312 tiles at M = 600, N = 13312 are 1 round + 56 tiles
+    ops, _ = _f8_ops(M=600, N=13312, K=1536)
+    g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
+    assert (g["waves"], g["nsplit"]) == ("4", "10880"), g
+    ops, _ = _f8_ops(M=130, N=16896, K=3072)                  # 132 tiles: one whole round
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
     assert (g["waves"], g["nsplit"]) == ("4", "0"), g
+    # where the planner runs the wide tile, the line is the wide tile's
+    for M, N, K, tile in [(512, 16640, 1024, ("256", "256", "8")), (512, 16384, 1024, ("256", "128", "8"))]:
+        ops, _ = _f8_ops(M=M, N=N, K=K)
+        g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
+        assert (g["bn"], g["bm"], g["waves"], g["nsplit"]) == tile + ("0",), g
     # few tiles: the narrowest tile spreads the work over more CUs
     ops, _ = _mx_ops(M=256, N=4096, K=1024)
     g = _geom(R.describe("gemm_nt_q_mxfp4", ops)[1])

@@ -407,16 +407,26 @@ def test_splitk_padded_views(gpu, row, dtype, M, N, K):
     assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["max_viol"] <= 1.0, c
 
 
-@pytest.mark.parametrize("rblk", [1, 128])
-def test_fp8_prefill_wide_tile_with_remainder(gpu, rblk):
+@pytest.mark.parametrize("M,N,K,rblk,n1", [(600, 13312, 1536, 1, 10880), (1200, 13312, 2048, 128, 13056)])
+def test_fp8_prefill_wide_tile_with_remainder(gpu, M, N, K, rblk, n1):
     """The e4m3 prefill's four-wave 128 x 256 tile over whole rounds of weight rows, and the
     remaining rows as a second launch on the 128 x 128 tile (both scale grids: the second
-    launch's weight-scale rows start n1 / rblk rows in)."""
-    M, N, K = 512, 16640, 1024
-    ops_desc = _f8_desc(M, N, K, rblk)
-    assert (ops_desc["waves"], ops_desc["nsplit"]) == ("4", "16384"), ops_desc
+    launch's weight-scale rows start n1 / rblk rows in), at shapes the 256-row tile leaves to
+    them: the rows about n1 and both ends against the oracle."""
+    gu = _gu()
+    d = _f8_desc(M, N, K, rblk)
+    assert (d["waves"], d["nsplit"]) == ("4", str(n1)) and "wide" not in d, d
     A, AS, B, BS = _f8_case(M, N, K, 77 + rblk, rblk)
-    _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk)
+    rc, Y, guards = gu.run_row(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu)
+    assert rc == R.RAD_OK and guards
+    assert (Y != gu.Y_SENTINEL).any(axis=0).all()          # every column written
+    for lo, hi in ((0, 256), (n1 - 256, min(n1 + 256, N)), (N - 256, N)):
+        b = BS[lo // rblk:-(-hi // rblk)]
+        Yr, Yf, S = O.quant_dot_fp8a8(A, AS, B[lo:hi], b, rblk, nthreads=16)
+        S8 = O.group8_mag("fp8a8", A, AS, B[lo:hi], b, rblk, nthreads=16)
+        c = gu.compare(np.ascontiguousarray(Y[:, lo:hi]), Yr, Yf, S, K, S8)
+        assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
+        assert c["max_viol"] <= 1.0 and c["rel_l2"] <= KBENCH_TOL["fp8a8"], c
 
 
 def _f8_desc(M, N, K, rblk):
