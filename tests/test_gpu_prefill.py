@@ -140,19 +140,20 @@ def test_mxfp4a16_short_scratch_refused(gpu):
     assert np.all(Y == _gu().Y_SENTINEL)                    # nothing launched
 
 
-F8_WIDE = [  # M, N, K, scratch: the fp8a8 wide tile, whole K and split
-    (1030, 8200, 128, None),      # 256 x 256: one step, six live tokens in the last tile, ragged N
-    (1030, 8448, 256, None),      # 256 x 256: two steps
-    (300, 21700, 384, None),      # 256 x 128: an odd step count, ragged M and N
-    (144, 300, 21504, "hook"),    # split: the least M, a ragged N past one tile
-    (260, 514, 5376, "hook"),     # split, N off a multiple of 4
-    (513, 300, 8192, "hook"),     # split, one live token in the last tile
-]
+F8_WIDE = [  # M, N, K, scratch, the tile's tokens, chunks: the fp8a8 wide tile, whole K and split
+    (1030, 8200, 128, None, 256, 1),      # one step, six live tokens in the last tile, ragged N
+    (1030, 8448, 256, None, 256, 1),      # two steps
+    (300, 21700, 384, None, 128, 1),      # an odd step count, ragged M and N
+    (144, 300, 21504, "hook", 128, 28),   # split: the least M, a ragged N past one tile
+    (260, 514, 5376, "hook", 128, 14),    # split, N off a multiple of 4
+    (513, 300, 8192, "hook", 128, 16),    # split, one live token in the last tile
+    (513, 3073, 13568, "hook", 256, 6),   # split of the larger tile: one live token and one live
+]                                         # row in the last ones, a shorter last chunk
 
 
 @pytest.mark.parametrize("scales", ["block", "channel", "vary", "late"])
-@pytest.mark.parametrize("M,N,K,scratch", F8_WIDE)
-def test_fp8_wide_tile(gpu, M, N, K, scratch, scales):
+@pytest.mark.parametrize("M,N,K,scratch,bm,kc", F8_WIDE)
+def test_fp8_wide_tile(gpu, M, N, K, scratch, bm, kc, scales):
     """The wide tile at its edges, on both scale grids; on the per-row grid with one scale a row
     (applied once after the walk), with scales that vary everywhere, and with one row's scale
     that differs in its last group alone (that row's tile must take the per-group walk)."""
@@ -164,24 +165,42 @@ def test_fp8_wide_tile(gpu, M, N, K, scratch, scales):
     if scales == "late":
         BS[N - 1, -1] += 0x80                              # twice as large
     A, AS, B, BS = (np.ascontiguousarray(t) for t in (A, AS, B, BS))
-    if not _wide_route(M, N, K, rblk, scratch):
-        pytest.skip("the planner keeps the base tiles at this shape and grid")
-    _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk, scratch=scratch)
+    g = _f8_geom(M, N, K, rblk, scratch)
+    assert (g["bm"], g.get("kc", "1")) == (str(bm), str(kc)), g
+    if M * N * K < 1 << 33:
+        _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, rblk=rblk, scratch=scratch)
+        return
+    gu = _gu()
+    rc, Y, ok = gu.run_row(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
+    assert rc == R.RAD_OK and ok and (Y != gu.Y_SENTINEL).any(axis=0).all()
+    for lo, hi in _ends(N):                                # the first and last rows' columns
+        b = BS[lo // rblk:-(-hi // rblk)]
+        Yr, Yf, S = O.quant_dot_fp8a8(A, AS, B[lo:hi], b, rblk, nthreads=16)
+        S8 = O.group8_mag("fp8a8", A, AS, B[lo:hi], b, rblk, nthreads=16)
+        _within(gu.compare(np.ascontiguousarray(Y[:, lo:hi]), Yr, Yf, S, K, S8))
 
 
-def _wide_route(M, N, K, rblk, scratch):
+def _ends(N):
+    return (0, 256), ((N - 200) // 128 * 128, N)
+
+
+def _within(c):
+    assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
+    assert c["max_viol"] <= 1.0, c
+
+
+def _f8_geom(M, N, K, rblk, scratch):
+    """describe's fields of a launch that the wide tile must take."""
     rows = N if rblk == 1 else (N + 127) // 128
     z = lambda *s, dt=torch.uint8: torch.zeros(s, dtype=dt)
     ops = R.GemmOperands(z(M, K), z(M, K // 128, dt=torch.float32), z(N, K),
                          z(rows, K // 128, dt=torch.int16), z(M, N, dt=torch.int16),
                          dtype="fp8a8", N=N, K=K)
     if scratch:
-        need = R.row_scratch_bytes("gemm_nt_q_fp8a8", ops)
-        if not need:
-            return False
-        ops.set_scratch(z(64), need)
+        ops.set_scratch(z(64), R.row_scratch_bytes("gemm_nt_q_fp8a8", ops))
     d = R.describe("gemm_nt_q_fp8a8", ops)[1]
-    return "kernel=f8wide" in d if scratch else "wide=" in d
+    assert ("kernel=f8wide" if scratch else "wide=") in d, d
+    return dict(f.split("=", 1) for f in d.split() if "=" in f)
 
 
 @pytest.mark.parametrize("bad", [0x7F80, 0x7FC0])
@@ -216,38 +235,56 @@ def test_fp8_wide_tile_large_token_scale(gpu, M, N, K, scratch):
         A[m], AS[m] = 0x7E, 1e31
     for n in (3, 300, N - 1):
         B[n], BS[n] = 0x7E, synth.bf16_bits(np.array([1e-10], np.float32))[0]
-    assert _wide_route(M, N, K, 1, scratch)
+    _f8_geom(M, N, K, 1, scratch)
     _, Y = _check(F8_TILE, "fp8a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
     assert np.isfinite(O.bf16_to_f32(Y)[:, [3, 300, N - 1]]).all()
 
 
-MX_SPLIT = [(144, 300, 8192), (260, 514, 5376), (513, 130, 6144)]   # M, N, K
+MX_SPLIT = [  # M, N, K, the tile's tokens, chunks
+    (144, 300, 8192, 128, 16), (260, 514, 5376, 128, 14), (513, 130, 6144, 128, 16),
+    (385, 3001, 8192, 256, 5)]            # 128 x 256: one live token, a shorter last chunk
 
 
-@pytest.mark.parametrize("M,N,K", MX_SPLIT)
-def test_mxfp4a8_prefill_splitk(gpu, M, N, K):
+def _mx_geom(row, ops, M, N, bm, kc):
+    g = dict(f.split("=", 1) for f in R.describe(row, ops)[1].split() if "=" in f)
+    assert (g["arm"], g["bn"], g["bm"], g["kc"]) == ("splitk", "128", str(bm), str(kc)), g
+    assert g["partials"] == str(4 * kc * M * N)
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("M,N,K,bm,kc", MX_SPLIT)
+def test_mxfp4a8_prefill_splitk(gpu, M, N, K, bm, kc, special):
     """K split past 128 tokens on the e2m1 tiles (ragged M and N, N off a multiple of 4, one
     live token in the last tile), against the bar of the unsplit tiles; a scratch one byte
-    short runs those."""
+    short runs those.  special: NaN codes, token scales and weight scales in the first and the
+    last chunk.  (Not Inf token scales: the oracle applies them to each 32-wide block, the MFMA
+    to a group's sum, and Inf - Inf is NaN in the former alone, split or not.)"""
     gu = _gu()
     A, AS, B, BS = _mx_case(M, N, K, M + N + K)
-    Yr, Yf, S = O.quant_dot_mxfp4a8(A, AS, B, BS, nthreads=16)
-    S8 = O.group8_mag("mxfp4a8", A, AS, B, BS, nthreads=16)
+    if special:
+        A[3, 5], A[M - 1, K - 1] = 0x7F, 0xFF
+        AS[7, 2], AS[11, -1] = np.nan, np.nan
+        BS[2, 1], BS[N - 1, -1] = 0xFF, 0xFF
     z = lambda *s, dt=torch.uint8: torch.zeros(s, dtype=dt)
     ops = R.GemmOperands(z(M, K), z(M, K // 128, dt=torch.float32), z(N, K // 2), z(N, K // 32),
                          z(M, N, dt=torch.int16), dtype="mxfp4a8", N=N, K=K)
     need = R.row_scratch_bytes(MX_TILE, ops)
-    assert need > 0 and need % (4 * M * N) == 0
+    assert need == 4 * kc * M * N
+    ops.set_scratch(z(64), need)
+    _mx_geom(MX_TILE, ops, M, N, bm, kc)
     for scratch in ("hook", None):
         rc, Y, guards = gu.run_row(MX_TILE, "mxfp4a8", A, AS, B, BS, M, N, K, gpu, scratch=scratch)
         assert rc == R.RAD_OK and guards
-        c = gu.compare(Y, Yr, Yf, S, K, S8)
-        assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
-        assert c["max_viol"] <= 1.0 and c["rel_l2"] <= 3e-2, c
+        for lo, hi in _ends(N) if N > 1024 else ((0, N),):
+            Yr, Yf, S = O.quant_dot_mxfp4a8(A, AS, B[lo:hi], BS[lo:hi], nthreads=16)
+            S8 = O.group8_mag("mxfp4a8", A, AS, B[lo:hi], BS[lo:hi], nthreads=16)
+            c = gu.compare(np.ascontiguousarray(Y[:, lo:hi]), Yr, Yf, S, K, S8)
+            _within(c)
+            assert c["rel_l2"] <= 3e-2, c
 
 
-@pytest.mark.parametrize("M,N,K", MX_SPLIT)
-def test_mxfp4a16_prefill_splitk(gpu, M, N, K):
+@pytest.mark.parametrize("M,N,K,bm,kc", MX_SPLIT)
+def test_mxfp4a16_prefill_splitk(gpu, M, N, K, bm, kc):
     """The same on the bf16-in row, whose hook asks for the planes past the quantised
     activations; with the activations' bytes alone, or one byte short of both, it runs
     unsplit."""
@@ -255,8 +292,6 @@ def test_mxfp4a16_prefill_splitk(gpu, M, N, K):
     X = _bf16_acts(M, K, M + N + K)
     B, BS = synth.mxfp4_weights(N, K, M + 3)
     Qr, SXr = O.quant_act_mxfp8(X)
-    Yr, Yf, S = O.dot_mx8_mxfp4(Qr, SXr, B, BS, nthreads=16)
-    S8 = O.group8_mag("mxfp4a16", Qr, SXr, B, BS, nthreads=16)
     base = ((M * K + 255) // 256) * 256 + M * (K // 32)
     gX, gB, gBS = gu.Guarded(X, gpu), gu.Guarded(B, gpu), gu.Guarded(BS, gpu)
     for short in (None, 1, 0):                             # whole, one byte short, no planes
@@ -264,19 +299,23 @@ def test_mxfp4a16_prefill_splitk(gpu, M, N, K):
         ops = R.GemmOperands(gX.t, None, gB.t, gBS.t, gY.t, dtype="mxfp4a16", N=N, K=K, group=32,
                              M=M)
         need = R.row_scratch_bytes(A16, ops)
-        planes = need - (base + 255) // 256 * 256
-        assert planes > 0 and planes % (4 * M * N) == 0
+        assert need - (base + 255) // 256 * 256 == 4 * kc * M * N
         nbytes = need if short is None else need - 1 if short else base
         gS = gu.Guarded(np.zeros(nbytes, np.uint8), gpu, fill=0x5A)
         ops.set_scratch(gS.t, nbytes)
-        arm = "arm=splitk" if short is None else "arm=prefill"
-        assert arm in R.describe(A16, ops)[1]
+        if short is None:
+            _mx_geom(A16, ops, M, N, bm, kc)
+        else:
+            assert "arm=prefill" in R.describe(A16, ops)[1]
         rc = R.launch_row(A16, ops, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert rc == R.RAD_OK and all(g.guards_intact() for g in (gX, gB, gBS, gY, gS))
         raw = gS.t.cpu().numpy()
         assert np.array_equal(raw[:M * K].reshape(M, K), Qr)
         Y = gY.t.cpu().numpy().view(np.uint16).reshape(M, N)
-        c = gu.compare(Y, Yr, Yf, S, K, S8)
-        assert c["sentinel_left"] == 0 and c["nan_mismatch"] == 0 and c["inf_mismatch"] == 0, c
-        assert c["max_viol"] <= 1.0 and c["row_rel_l2_max"] <= 2.0 ** -8, c
+        for lo, hi in _ends(N) if N > 1024 else ((0, N),):
+            Yr, Yf, S = O.dot_mx8_mxfp4(Qr, SXr, B[lo:hi], BS[lo:hi], nthreads=16)
+            S8 = O.group8_mag("mxfp4a16", Qr, SXr, B[lo:hi], BS[lo:hi], nthreads=16)
+            c = gu.compare(np.ascontiguousarray(Y[:, lo:hi]), Yr, Yf, S, K, S8)
+            _within(c)
+            assert c["row_rel_l2_max"] <= 2.0 ** -8, c
