@@ -125,26 +125,61 @@ def test_logits_parity(gpu, M, N, K, sdt, br, xp, yp):
     check(Y, x, codes, sbits, sdt, br, "logits_M%d_N%d_K%d_%s_br%d" % (M, N, K, sdt, br))
 
 
-WIDE = [  # M, N, K, sdt, br, x_pitch, y_pitch: the wide walk (9 rows up, 16384 head rows up)
-    (9, 16384, 256, "bf16", 1, None, None),      # one window, the smallest head
-    (16, 16387, 144, "f16", 1, None, None),      # ragged N and a 16-wide last scale block
-    (17, 16500, 400, "bf16", 128, 408, 16501),   # two groups, odd logits pitch: scalar stores
-    (33, 16640, 272, "f32", 1, None, 16644),     # three groups
-    (64, 16385, 640, "bf16", 1, None, None),     # four groups, a block with one live row
-    (70, 16401, 208, "f32", 128, None, None),    # a second pass of six rows
-    (12, 65600, 512, "bf16", 1, None, None),     # one-tile blocks, more blocks than workgroups
-    (40, 131072, 256, "bf16", 1, None, None),    # two-tile blocks, one each
+WIDE = [  # M, N, K, sdt, br, x_pitch, y_pitch, walk, most blocks a workgroup: the wide walk (9
+          # rows up, 16384 head rows up)
+    (9, 16384, 256, "bf16", 1, None, None, "wide1", 1),      # one window, the smallest head
+    (16, 16387, 144, "f16", 1, None, None, "wide1", 1),      # ragged N, a 16-wide last scale block
+    (17, 16500, 400, "bf16", 128, 408, 16501, "wide1", 1),   # two groups, odd logits pitch: scalar stores
+    (33, 16640, 272, "f32", 1, None, 16644, "wide1", 1),     # three groups
+    (64, 16385, 640, "bf16", 1, None, None, "wide1", 1),     # four groups, a block with one live row
+    (70, 16401, 208, "f32", 128, None, None, "wide1", 1),    # a second pass of six rows
+    (12, 65600, 512, "bf16", 1, None, None, "wide1", 2),     # 513 blocks of one tile on 512 workgroups
+    (40, 131072, 256, "bf16", 1, None, None, "wide2", 1),    # two-tile blocks, one each
+    # several blocks a workgroup: cursors, sums and stores cross them, after an odd window count
+    # (the double buffers' parity changes there) and an even one
+    (16, 151930, 528, "bf16", 1, None, None, "wide1", 3),
+    (9, 151936, 208, "bf16", 128, None, None, "wide1", 3),
+    (16, 262144, 144, "f32", 1, None, None, "wide2", 2),
+    (50, 262100, 272, "bf16", 1, None, None, "wide2", 2),
 ]
 
 
-@pytest.mark.parametrize("M,N,K,sdt,br,xp,yp", WIDE)
-def test_logits_wide_parity(gpu, M, N, K, sdt, br, xp, yp):
+@pytest.mark.parametrize("M,N,K,sdt,br,xp,yp,walk,deep", WIDE)
+def test_logits_wide_parity(gpu, M, N, K, sdt, br, xp, yp, walk, deep):
     print("logits wide parity M=%d N=%d K=%d %s br=%d" % (M, N, K, sdt, br), flush=True)
     codes, sbits = LU.head(N, K, M * 7 + N, sdt, br)
     x = synth.bf16_bits(np.random.default_rng(M + K).standard_normal((M, K)).astype(np.float32))
+    _wide_desc(M, N, K, sdt, br, walk, deep)
     rc, Y, ok = run(x, codes, sbits, sdt, br, gpu, xp, yp)
     assert rc == R.RAD_OK and ok
     check(Y, x, codes, sbits, sdt, br, "logits_wide_M%d_N%d_K%d_%s_br%d" % (M, N, K, sdt, br))
+
+
+def _wide_desc(M, N, K, sdt, br, walk, deep):
+    from tests.test_logits import _desc, _ops
+    g = _desc(_ops(M=M, N=N, K=K, sdt=sdt, br=br)[0])[1]
+    assert (g["walk"], -(-int(g["chunks"]) // int(g["blocks"]))) == (walk, deep), g
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 33000, 400), (40, 70000, 256)])
+def test_wide_special_values_poison_their_rows(gpu, M, N, K):
+    """NaN codes and scales, NaN and Inf activations through the wide walk, in the first and last
+    head rows and columns: NaN and Inf where the oracle has them alone.  (Not Inf scales: the
+    oracle scales each product, the kernel the sum of a block.)"""
+    _wide_desc(M, N, K, "bf16", 1, "wide2", 1)
+    codes, sbits = LU.head(N, K, 3)
+    codes[5, 17], codes[N - 1, K - 1] = 0x7F, 0xFF
+    sbits[9, 0], sbits[N - 3, -1] = 0x7FC0, 0xFFC1
+    x = synth.bf16_bits(np.random.default_rng(1).standard_normal((M, K)).astype(np.float32))
+    x[2, 3], x[M - 1, K - 1] = 0x7FC0, 0x7F80
+    rc, Y, ok = run(x, codes, sbits, "bf16", 1, gpu)
+    assert rc == R.RAD_OK and ok
+    Yo, _ = O.logits_e4m3(x, codes, sbits, "bf16", 1)
+    assert np.isnan(Y[:, [5, 9, N - 3, N - 1]]).all() and np.isnan(Y[2]).all()
+    rows = [m for m in range(M) if m not in (2, M - 1)]
+    cols = np.setdiff1d(np.arange(N), [5, 9, N - 3, N - 1])
+    assert np.isfinite(Y[rows][:, cols]).all()
+    assert np.array_equal(np.isnan(Y), np.isnan(Yo)) and np.array_equal(np.isinf(Y), np.isinf(Yo))
 
 
 @pytest.mark.parametrize("sdt,br,pad,shift", [("bf16", 1, 3, 0), ("f16", 1, 0, 2),
@@ -196,12 +231,12 @@ def test_nan_code_and_scale_poison_their_rows(gpu):
     check(Y, x, codes, sbits, "bf16", 1, "logits_nan_codes")
 
 
-def test_header_cache_and_guard(gpu):
+@pytest.mark.parametrize("M,N,K", [(2, 300, 256), (16, 16500, 256)])   # 4-row walk, wide walk
+def test_header_cache_and_guard(gpu, M, N, K):
     """The first launch over a device blob caches its header.  A different head joined at
     the same address (scale rows per 128 instead of per row) without forgetting it: the
     kernel's check of the device header fails and every logit is NaN (never a read past
     the planes); after forget_head the launch reads the new header and is right."""
-    M, N, K = 2, 300, 256
     x = synth.bf16_bits(np.random.default_rng(2).standard_normal((M, K)).astype(np.float32))
     c1, s1 = LU.head(N, K, 4, "bf16", 1)
     c2, s2 = LU.head(N, K, 5, "bf16", 128)
