@@ -49,7 +49,7 @@ constexpr int prefill_stage_bytes(int wnf, int wmw, int wh = 1, int wv = 8) {
 template <int WMW>
 struct PrefillF8Layout {
     static constexpr int BN = 256, BM = 32 * WMW;
-    static constexpr int WLD = BN / 64, ALD = BM / 64, LOADS = WLD + ALD + 2;
+    static constexpr int WLD = BN / 64, ALD = BM / 64;   /* plane loads a wave */
     static constexpr int W = 0;                   /* [BN/16][2 halves][1 KB] weights */
     static constexpr int S = W + BN * 128;        /* [256] dwords: a weight row's bf16 scale */
     static constexpr int A = S + 1024;            /* [BM/16][2 halves][1 KB] activations */

@@ -284,14 +284,14 @@ def _wide_split(N, K, M, mx, units=256, min_steps=4):
 
 def test_tile_splitk_hook_and_arm():
     """The tile rows' scratch hook sizes split K's f32 partial planes (kc * M * N * 4) up to
-    M = 128 on a narrow N and returns 0 elsewhere; with that scratch the launch describes
-    the split arm, with less (or misaligned) the unsplit arms it had before."""
+    M = 128 on a narrow N (past it: test_prefill_splitk_hook_and_arm); with that scratch the
+    launch describes the split arm, with less (or misaligned) the unsplit arms it had before."""
     rows = {r["name"]: r for r in R.rows()}
     assert rows["gemm_nt_q_mxfp4"]["scratch"] and rows["gemm_nt_q_fp8a8"]["scratch"]
     # up to M = 64 the skinny-band GEMV over 256-row tiles, else the 128 x 128 tile.  Config 2
     # at M = 64: down 21 tiles x 12 chunks of 14 groups, qkv 32 x 7 of 6, gate_up 84 x 3 of
     # 14 (both encodings); past M = 64 down splits 42 x 6 of 28 and gate_up's 168 tiles fill
-    # the chip unsplit; M past 128 and one-chunk K never split
+    # the chip unsplit; M = 129..143 and one-chunk K never split
     assert _wide_split(5376, 21504, 64, True) == (12, 14) == _wide_split(5376, 21504, 64, False)
     assert _wide_split(8192, 5376, 64, True) == (7, 6)
     assert _wide_split(21504, 5376, 64, False) == (3, 14)
@@ -334,6 +334,40 @@ def test_tile_splitk_hook_and_arm():
         ops = R.GemmOperands(a, s, b, bs, None, dtype="mxfp4a8", N=5376, K=21504,
                              extra_params=extra)
         assert R.row_scratch_bytes("gemm_nt_q_mxfp4", ops) == (6 if M > 64 else 12) * M * 5376 * 4
+
+
+@pytest.mark.parametrize("row,M,N,K", [
+    (row, M, N, K) for row in ("gemm_nt_q_mxfp4", "gemm_nt_q_fp8a8", "gemm_nt_q_mxfp4a16")
+    # the narrowest and a wide N, a K of prime group count, a large M, the largest planes
+    for M, N, K in [(144, 128, 5376), (144, 5376, 21504), (200, 300, 3968), (700, 2000, 8576),
+                    (2048, 512, 8192), (512, 5376, 21504), (1000, 2000, 21504)]])
+def test_prefill_splitk_hook_and_arm(row, M, N, K):
+    """From M = 144 the tile rows and the bf16-in row split K where their costs say so: the hook
+    asks for kc planes (past the quantised activations at mxfp4a16), every chunk has a step, no
+    two workgroups wait for a third round, and a byte less runs unsplit; one row of tokens fewer
+    than 144 never splits."""
+    a16 = row == "gemm_nt_q_mxfp4a16"
+    def ops_of(m):
+        if a16:
+            return _a16_ops(M=m, N=N, K=K, scratch=False)[0]
+        return (_mx_ops if row == "gemm_nt_q_mxfp4" else _f8_ops)(M=m, N=N, K=K)[0]
+    base = lambda m: ((m * K + 255) // 256 * 256 + m * (K // 32)) if a16 else 0
+    assert R.row_scratch_bytes(row, ops_of(143)) == base(143)
+    ops = ops_of(M)
+    need = R.row_scratch_bytes(row, ops)
+    off = (base(M) + 255) // 256 * 256
+    kc, rest = divmod(need - off, 4 * M * N)
+    assert kc >= 2 and rest == 0
+    sc = FakeT(_aligned((64,), np.uint8))
+    ops.set_scratch(sc, need)
+    g = _geom(R.describe(row, ops)[1])
+    assert (g["arm"], g["kc"], g["partials"]) == ("splitk", str(kc), str(need - off)), g
+    cst, steps, tiles = int(g["cst"]), K // 128, int(g["tiles"])
+    assert (kc - 1) * cst < steps <= kc * cst and cst >= 3, g
+    assert tiles * kc <= 512 and need - off <= 256 << 20, g
+    assert tiles == -(-N // int(g["bn"])) * -(-M // int(g["bm"])), g
+    ops.set_scratch(sc, need - 1)
+    assert _geom(R.describe(row, ops)[1])["arm"] == "prefill"
 
 
 @pytest.mark.parametrize("M,N,K,tw", [
