@@ -94,8 +94,21 @@ class Capture:
     def present(self, i):
         return i < len(self.tensors) and not self.tensors[i]["null"]
 
-    def truncated(self):
-        return any(t["trunc"] for t in self.tensors) or (self.scratch and self.scratch[2])
+    def operand_cut(self):
+        return any(t["trunc"] for t in self.tensors)
+
+    def scratch_cut(self):
+        """The scratch was cut before the end of what the oracle's check reads of it: the
+        quantised activations, or the gate_up plane (a K split's planes are read by none)."""
+        if not self.scratch or not self.scratch[2]:
+            return False
+        need, N, K = 0, self.geti("N"), self.geti("K")
+        if self.row.startswith("gemm_nt_q_gated"):
+            need = 4 * numel(self.tensors[4])                  # [M, N] bf16, [M, N / 2] codes
+        elif self.row.startswith("gemm_nt_q") and self.gets("dtype") == "mxfp4a16":
+            M = numel(self.tensors[4]) // N
+            need = (M * K + 255) // 256 * 256 + M * (K // 32)
+        return self.scratch[1] < need
 
 
 def row_stride(t, cols):
@@ -375,6 +388,15 @@ def replay_oracle(c):
     return False, "no oracle for row %s" % c.row
 
 
+def launch_scratch(c, dev):
+    """Scratch of the captured launch's size: the bytes captured, zeros past a cut (a launch
+    writes what it reads of its scratch, so those are no input of it)."""
+    import torch
+    buf = torch.zeros(c.scratch[0], dtype=torch.uint8, device=dev)
+    buf[:c.scratch[1]] = torch.from_numpy(np.ascontiguousarray(c.pre[-1])).to(dev)
+    return buf
+
+
 def replay_device(c):
     """Re-launch the capture through the library on cuda:0; outputs must equal POST."""
     import ctypes
@@ -406,10 +428,7 @@ def replay_device(c):
         kb = k.encode()
         keep.append(kb)
         tv[i].name, tv[i].value = kb, v
-    scratch = None
-    if c.scratch:
-        scratch = torch.from_numpy(np.ascontiguousarray(c.pre[-1])).to(dev) if c.scratch[1] \
-            else torch.zeros(c.scratch[0], dtype=torch.uint8, device=dev)
+    scratch = launch_scratch(c, dev) if c.scratch else None
     args = R.RadArgs(ctypes.cast(t, ctypes.POINTER(R.RadTensor)), len(c.tensors),
                      ctypes.cast(p, ctypes.POINTER(R.RadParam)), len(c.params),
                      ctypes.cast(tv, ctypes.POINTER(R.RadTunableValue)), len(c.tunables),
@@ -459,7 +478,7 @@ def main(argv=None):
         if c.post is None and not args.device:
             print("%s  %s: refused (status %d), nothing to compare" % (os.path.basename(d), c.row, c.rc))
             continue
-        if c.truncated() and not args.device:
+        if c.operand_cut() or (c.scratch_cut() and not args.device):
             print("%s  %s: an operand was cut at R3D_DUMP_CAP, not replayed" % (os.path.basename(d), c.row))
             continue
         ok, msg = replay_device(c) if args.device else replay_oracle(c)

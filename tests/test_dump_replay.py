@@ -14,9 +14,9 @@ from tests import replay_dump as RD
 DT = RD.DT
 
 
-def write_capture(d, row, params, tensors, pre, post, scratch=None, rc=0):
-    """tensors: [(dtype name, shape, stride) or None]; pre/post: per-operand byte arrays
-    (+ the scratch span last when scratch = (bytes, captured))."""
+def write_capture(d, row, params, tensors, pre, post, scratch=None, rc=0, cut=()):
+    """tensors: [(dtype name, shape, stride) or None]; pre/post: per-operand byte arrays (cut where
+    `cut` names the operand; + the scratch span last when scratch = (bytes, captured))."""
     os.makedirs(d, exist_ok=True)
     with open(os.path.join(d, "manifest.tsv"), "w") as f:
         f.write("H\t%s\t%d\t%d\t%d\n" % (row, rc, len(tensors), len(params)))
@@ -32,11 +32,11 @@ def write_capture(d, row, params, tensors, pre, post, scratch=None, rc=0):
                 f.write("T\t%d\t0\t0\t0\t0\t1\t0x0\n" % i)
                 continue
             name, shape, stride = t
-            f.write("T\t%d\t%d\t%d\t%s\t%s\t%d\t0\t0\t0x1000\n" % (
+            f.write("T\t%d\t%d\t%d\t%s\t%s\t%d\t%d\t0\t0x1000\n" % (
                 i, DT[name], len(shape), "\t".join(map(str, shape)), "\t".join(map(str, stride)),
-                pre[i].size))
+                pre[i].size, i in cut))
         if scratch:
-            f.write("X\t%d\t%d\t0\n" % scratch)
+            f.write("X\t%d\t%d\t%d\n" % (scratch + (scratch[1] < scratch[0],)))
     for name, spans in (("pre.bin", pre), ("post.bin", post)):
         with open(os.path.join(d, name), "wb") as g:
             for s in spans:
@@ -95,6 +95,57 @@ def test_mxfp4_gemm_capture_replays_within_bound(tmp_path, pad):
                   pre, [a_span, b(AS), b(B), b(BS), b(bad), None, None])
     res = [RD.replay_oracle(RD.Capture(c)) for c in RD.captures([str(tmp_path)])]
     assert res[0][0] and not res[1][0], res
+
+
+@pytest.mark.parametrize("dtype", ["mxfp4a8", "mxfp4a16"])
+def test_capture_with_cut_split_planes_replays(tmp_path, capsys, dtype):
+    """A K split's scratch is larger than a capture keeps.  The cut planes are no input of a
+    check: the capture replays (mxfp4a16: as long as the quantised activations ahead of them are
+    whole), and a launch of it gets scratch of the recorded size, not of the captured one.  With
+    an operand cut, neither."""
+    rng = np.random.default_rng(3)
+    M, N, K = 2, 40, 256
+    a16 = dtype == "mxfp4a16"
+    B, BS = synth.mxfp4_weights(N, K, 4)
+    if a16:
+        X = synth.bf16_bits(rng.standard_normal((M, K)).astype(np.float32))
+        Q, SX = O.quant_act_mxfp8(X)
+        Yr, _, _ = O.dot_mx8_mxfp4(Q, SX, B, BS)
+        head = np.concatenate([b(Q), b(SX)])               # M K is a multiple of 256
+        first, a_s, asp = ("BF16", [M, K], [K, 1]), None, None
+        ab = b(X)
+    else:
+        _, A, AS = synth.activations(M, K, 3)
+        Yr, _, _ = O.quant_dot_mxfp4a8(A, AS, B, BS)
+        head = np.zeros(0, np.uint8)
+        first, a_s, asp = ("F8E4M3", [M, K], [K, 1]), ("F32", [M, 2], [2, 1]), b(AS)
+        ab = b(A)
+    ten = [first, a_s, ("FP4E2M1", [N, K], [K, 1]), ("E8M0", [N, K // 32], [K // 32, 1]),
+           ("BF16", [M, N], [N, 1]), None, None]
+    row = "gemm_nt_q_mxfp4a16" if a16 else "gemm_nt_q_mxfp4"
+    params = [("dtype", dtype), ("N", N), ("K", K), ("group", 32), ("M", M)]
+    whole, kept = 100000, 4096
+    sc = np.concatenate([head, rng.integers(0, 256, kept - head.size, dtype=np.uint8)])
+
+    def write(name, n, **kw):
+        write_capture(tmp_path / name, row, params, ten,
+                      [ab, asp, b(B), b(BS), np.zeros(M * N * 2, np.uint8), None, None, sc[:n]],
+                      [ab, asp, b(B), b(BS), b(Yr), None, None, sc[:n]], scratch=(whole, n), **kw)
+        return RD.Capture(str(tmp_path / name))
+
+    c = write("0000_" + row, kept)
+    assert not c.operand_cut() and not c.scratch_cut()
+    assert RD.replay_oracle(c)[0] and RD.main([c.dir]) == 0
+    assert "not replayed" not in capsys.readouterr().out
+    buf = RD.launch_scratch(c, "cpu")
+    assert buf.numel() == whole and np.array_equal(buf[:kept].numpy(), sc) and not buf[kept:].any()
+    c = write("0001_" + row, 256)                          # short of the codes' scales
+    assert c.scratch_cut() == a16
+    c = write("0002_" + row, kept, cut=(2,))
+    assert c.operand_cut()
+    for mode in ([], ["--device"]):                        # neither checked nor launched
+        assert RD.main([c.dir] + mode) == 0
+        assert "not replayed" in capsys.readouterr().out
 
 
 def test_rmsnorm_capture_with_residual_replays_exact(tmp_path):
