@@ -183,9 +183,10 @@ void r3d_gfx950_logits_head_forget(const void* blob);
 /* gemm_nt_q at dtype "mxfp4a16" that allocates nothing: no counterpart in the reference,
  * for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same operands, parameters, kernels and results as
- * r3d_rad_gemm_nt_q_mxfp4a16, but RadArgs::scratch is not used: the quantised activations
- * go to a static device buffer of R3D_NOALLOC_SCRATCH_BYTES per GPU, held until the
- * process ends.  A call needing more (round256(M*K) + M*K/32 bytes) is refused with
+ * r3d_rad_gemm_nt_q_mxfp4a16 with R3D_NOALLOC_SCRATCH_BYTES of scratch, but RadArgs::scratch
+ * is not used: the quantised activations, and a K split's planes where they fit behind them
+ * (else the launch runs unsplit, its sums rounded in another order), go to a static device
+ * buffer of that size per GPU, held until the process ends.  A call needing more (round256(M*K) + M*K/32 bytes) is refused with
  * RAD_E_SHAPE and a line on stderr.  All calls on one GPU share its buffer: calls that
  * overlap on one GPU (other streams, other threads) race. */
 #define R3D_NOALLOC_SCRATCH_BYTES (16ll << 20)

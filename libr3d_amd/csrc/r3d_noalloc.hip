@@ -6,9 +6,11 @@
  * E8M0 scales) before the GEMM reads them.  This entry runs the same kernels with that
  * scratch in a file-scope device array of R3D_NOALLOC_SCRATCH_BYTES: each GPU the library
  * runs on holds its own copy until the process ends, and the entry allocates and frees
- * nothing.  Every call on one GPU shares that GPU's array, so calls that overlap on one
- * GPU (two streams, two threads) race on it; calls in one stream order are safe.  The
- * quantiser writes every byte the GEMM then reads, so nothing has to start at zero.
+ * nothing.  A K split's planes use what the activations leave of it; where they do not fit,
+ * the launch runs unsplit, as the row does with that much scratch.  Every call on one GPU
+ * shares that GPU's array, so calls that overlap on one GPU (two streams, two threads) race on
+ * it; calls in one stream order are safe.  The quantiser and the split write every byte that
+ * is then read, so nothing has to start at zero.
  */
 #include <hip/hip_runtime.h>
 

@@ -1,6 +1,6 @@
 """r3d_rad_gemm_nt_q_mxfp4a16_noalloc (run by pytest last): the mxfp4a16 row with its quantiser scratch in a
 static device buffer instead of RadArgs::scratch.  Through the C ABI it must give exactly
-the bytes of the allocating row on the same operands, on two calls in a row (the second
+the bytes of the row with as much scratch on the same operands, on two calls in a row (the second
 smaller, over the first call's leftovers), refuse a call whose scratch need passes the
 buffer (RAD_E_SHAPE, nothing launched), and leave the device's free memory unchanged."""
 import ctypes
@@ -54,6 +54,37 @@ def test_noalloc_matches_allocating_row_twice(gpu):
         ref, got = _run_both(M, N, K, seed, gpu)
         assert np.array_equal(ref, got), (M, N, K, int(np.sum(ref != got)))
         assert not np.any(got == 0x7777)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,fits", [(144, 300, 8192, True), (385, 3001, 8192, False)])
+def test_noalloc_splits_where_the_planes_fit(gpu, M, N, K, fits):
+    """The entry is the row with the static buffer's size of scratch: the K split where its
+    planes fit behind the quantised activations, else the unsplit launch."""
+    from tests import gpu_util as gu
+    x, b, bs = _operands(M, N, K, 14, gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def row(nbytes):
+        y = torch.full((M, N), 0x7777, dtype=torch.int16, device=gpu)
+        ops = R.GemmOperands(x, None, b, bs, y, dtype="mxfp4a16", N=N, K=K, group=32, M=M)
+        need = R.row_scratch_bytes(A16, ops)
+        nbytes = need if nbytes is None else nbytes
+        ops.set_scratch(torch.empty(nbytes, dtype=torch.uint8, device=gpu), nbytes)
+        assert R.launch_row(A16, ops, stream) == R.RAD_OK
+        torch.cuda.synchronize()
+        return need, y.cpu().numpy()
+
+    need, split = row(None)
+    assert (need <= 16 << 20) == fits
+    gY = gu.y_buffer(M, N, gpu)
+    ops = R.GemmOperands(x, None, b, bs, gY.t, dtype="mxfp4a16", N=N, K=K, group=32, M=M)
+    assert _noalloc()(ctypes.byref(ops.args), ctypes.c_void_p(stream)) == R.RAD_OK
+    torch.cuda.synchronize()
+    assert gY.guards_intact()
+    got = gY.t.cpu().numpy()
+    assert np.array_equal(got, row(16 << 20)[1])
+    assert np.array_equal(got, split) == fits              # the two orders round apart
 
 
 @pytest.mark.gpu
