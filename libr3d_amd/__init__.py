@@ -798,7 +798,11 @@ def gemm_nt_q(a, a_scale, b, b_scale, y, *, dtype, N, K, group=None, stream=None
         row = r["name"]
     need = row_scratch_bytes(row, ops)
     if need > 0:                        # the row's hook sized it, as an engine's arena would
-        ops.set_scratch(torch.empty(need, dtype=torch.uint8, device=y.device), need)
+        # from the launch stream's pool: it is freed on return, and whatever takes the memory
+        # next must come after the launch
+        own = None if stream is None else torch.cuda.ExternalStream(stream, device=y.device)
+        with torch.cuda.stream(own):
+            ops.set_scratch(torch.empty(need, dtype=torch.uint8, device=y.device), need)
     if stream is None:
         stream = torch.cuda.current_stream().cuda_stream
     return launch_row(row, ops, stream), row

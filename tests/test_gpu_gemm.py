@@ -438,6 +438,35 @@ def _f8_desc(M, N, K, rblk):
     return _geom(R.describe(F8_TILE, ops)[1])
 
 
+def test_gemm_nt_q_scratch_belongs_to_its_stream(gpu, monkeypatch):
+    """gemm_nt_q on another stream than the current one: its scratch, free again when it returns,
+    must not be what the current stream's next allocation gets (the launch still writes it), and
+    the next call on that stream may have it.  Then the call itself, against the current
+    stream's."""
+    import torch
+    M, N, K = 300, 514, 8192
+    A, AS, B, BS = (torch.from_numpy(t).to(gpu) for t in _mx_case(M, N, K, 5))
+    y = torch.zeros((M, N), dtype=torch.int16, device=gpu)
+    side = torch.cuda.Stream()
+    seen = []
+    with monkeypatch.context() as m:
+        m.setattr(R, "launch_row", lambda row, ops, st: seen.append(
+            (ops.args.scratch, ops.args.scratch_bytes, st)) or R.RAD_OK)
+        for _ in range(2):
+            assert R.gemm_nt_q(A, AS, B, BS, y, dtype="mxfp4a8", N=N, K=K,
+                               stream=side.cuda_stream)[0] == R.RAD_OK
+    ptr, need, st = seen[0]
+    assert need > 0 and st == side.cuda_stream and seen[1][0] == ptr
+    taken = [torch.empty(need, dtype=torch.uint8, device=gpu) for _ in range(4)]
+    assert all(t.data_ptr() != ptr for t in taken)
+    torch.cuda.synchronize()
+    assert R.gemm_nt_q(A, AS, B, BS, y, dtype="mxfp4a8", N=N, K=K, stream=side.cuda_stream)[0] == R.RAD_OK
+    y2 = torch.zeros_like(y)
+    assert R.gemm_nt_q(A, AS, B, BS, y2, dtype="mxfp4a8", N=N, K=K)[0] == R.RAD_OK
+    torch.cuda.synchronize()
+    assert y.any() and torch.equal(y, y2)
+
+
 def test_splitk_short_scratch_runs_unsplit(gpu):
     """A byte short of the hook's size: the launch takes the unsplit arm, leaves the
     scratch untouched (its poison and red zones intact) and still meets the bar."""
