@@ -136,8 +136,9 @@ static int launch_quad(const GemmPlan& P, const QuadGeom& g, hipStream_t stream)
     return RAD_OK;
 }
 
-/* passes > 1: P.M = 17..64 rows in 16-row passes side by side (grid.y), each pass exactly a
- * 16-row call's arithmetic; g is the 16-row geometry */
+/* passes > 1: P.M = 17..64 rows in 16-row passes, neighbours in grid.x over a weight block
+ * (the kernel's prologue); g is the 16-row geometry that lines_geom gives that many passes
+ * (its chunks may differ from a 16-row call's, and with them the order of a sum) */
 static int launch_lines(const GemmPlan& P, const LinesGeom& g, hipStream_t stream,
                         int passes = 1) {
     if (forced_fail(passes > 1 ? "skinny" : "lines"))
@@ -392,7 +393,7 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
     if ((P.ua & UA_GEMM) && mode != PF_MX8)
         return launch_any(P, mode, P.A, P.AS, P.a_pitch, P.as_pitch, stream);
     int cst = 0;
-    PrefillGeom gs{};                                    /* the split's tile (kind 2) */
+    PrefillGeom gs{};                                    /* the split's tile (kinds 2 to 4) */
     WideGeom gw{};                                       /* or its GEMV (kind 1) */
     int kc = 0;
     const int kind = part && ((uintptr_t)part & 15) == 0 && !P.ua
@@ -400,8 +401,8 @@ static int launch_prefill(const GemmPlan& P, hipStream_t stream, int stage = 0,
                          : 0;
     const bool split = kind != 0 && part_bytes >= (int64_t)kc * P.M * P.N * 4 &&
                        (kind != 2 || (gs.grid_m == 1 && gs.tiles * kc <= 0x7FFFFFFF));
-    /* the skinny band on a narrow N: 16-row passes of the decode GEMVs (each output row is
-     * the same arithmetic either way) */
+    /* the skinny band on a narrow N: 16-row passes of the decode GEMVs, in one launch where the
+     * line GEMV serves them */
     if (const int passes = split || P.ua ? 0 : skinny_passes(P.enc, P.M, P.N, cu_count())) {
         GemmPlan S = P;
         S.M = 16;
@@ -761,23 +762,26 @@ static int rms_entry(const RadArgs* a, RadStream s) {
      *   n = 1024   M = 4 4.3 -> 4.2 (512, 1), 4096 13.5 -> 12.8 (256, 1) */
     const int64_t nc = P.n / 8;
     const bool few = P.rows <= 512;
-    const int shape = !vq || P.g != 128 ? 0
-                    : nc <= 256 ? (few ? 5121 : 2561)
-                    : nc <= 512 ? (P.rows <= 1536 ? 5121 : 0)
-                    : nc <= 768 ? (few ? 10241 : 2563)
-                    : nc <= 1024 ? (few ? 10241 : 5122)
-                    : nc <= 2048 && few ? 10242 : 0;
+    struct { int lanes, chunks; } reg = {0, 0};          /* lanes 0: not held in registers */
+    if (vq && P.g == 128) {
+        if (nc <= 256) reg = {few ? 512 : 256, 1};
+        else if (nc <= 512) reg = {P.rows <= 1536 ? 512 : 0, 1};
+        else if (nc <= 768) reg = {few ? 1024 : 256, few ? 1 : 3};
+        else if (nc <= 1024) reg = {few ? 1024 : 512, few ? 1 : 2};
+        else if (nc <= 2048 && few) reg = {1024, 2};
+    }
 #define R3D_RMR(W_, T_, U_)                                                                 \
     hipLaunchKernelGGL((rmsnorm_quant_fp8_reg_kernel<W_, T_, U_>), dim3((unsigned)P.rows),    \
                        dim3(T_), 0, stream, reinterpret_cast<const uint16_t*>(P.x), P.x_pitch, \
                        reinterpret_cast<uint16_t*>(P.res), P.r_pitch, P.w, P.q, P.q_pitch,     \
                        P.scale, P.s_pitch, P.ob, P.ob_bf16, P.ob_pitch, (int)P.n, P.eps, P.wadd)
 #define R3D_RMRS(W_)                                                                        \
-    switch (shape) {                                                                        \
-        case 2561: R3D_RMR(W_, 256, 1); break;   case 2563: R3D_RMR(W_, 256, 3); break;     \
-        case 5121: R3D_RMR(W_, 512, 1); break;   case 5122: R3D_RMR(W_, 512, 2); break;     \
-        case 10241: R3D_RMR(W_, 1024, 1); break; default: R3D_RMR(W_, 1024, 2); break;      \
-    }
+    if (reg.lanes == 256 && reg.chunks == 1) { R3D_RMR(W_, 256, 1); }                       \
+    else if (reg.lanes == 256) { R3D_RMR(W_, 256, 3); }                                     \
+    else if (reg.lanes == 512 && reg.chunks == 1) { R3D_RMR(W_, 512, 1); }                  \
+    else if (reg.lanes == 512) { R3D_RMR(W_, 512, 2); }                                     \
+    else if (reg.chunks == 1) { R3D_RMR(W_, 1024, 1); }                                     \
+    else { R3D_RMR(W_, 1024, 2); }
 #define R3D_RMS(W_, V_, L_)                                                                 \
     hipLaunchKernelGGL((rmsnorm_quant_fp8_kernel<W_, V_, L_>), dim3((unsigned)P.rows),        \
                        dim3(256), lds, stream, reinterpret_cast<const uint16_t*>(P.x),        \
@@ -793,7 +797,7 @@ static int rms_entry(const RadArgs* a, RadStream s) {
         case 16: R3D_RMS(W_, true, 16); break; case 32: R3D_RMS(W_, true, 32); break;       \
         default: R3D_RMS(W_, true, 64); break;                                              \
     }
-    if (shape) {
+    if (reg.lanes) {
         if (P.w_bf16) { R3D_RMRS(true) } else { R3D_RMRS(false) }
     } else if (P.w_bf16) { R3D_RMSL(true) } else { R3D_RMSL(false) }
 #undef R3D_RMSL

@@ -70,7 +70,7 @@ struct LinesUnit {
 };
 
 /* The small parameters packed into one argument: M (1..64: the skinny band's passes see
- * up to 16 each) in bits 0-6, log2 of the chunk count (0..4) in bits 7-9, fp8a8 weight
+ * up to 16 each) in bits 0-6, log2 of the chunk count (0..3) in bits 7-9, fp8a8 weight
  * scales on the 128 x 128 block grid in bit 10, a_scale rows at a pitch of K / 128 floats
  * in bit 11. */
 constexpr int lines_pack(int M, int log2_chunks, bool rblk128, bool as_dense) {
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64 * WV) void gemv_lines_kernel(
     const bool rblk128 = (pk >> 10) & 1, as_dense = (pk >> 11) & 1;
     const int groups = K >> 7;
     /* M > 16 (the skinny band): pass y computes activation rows [16 y, 16 y + 16) of a taller
-     * A -- the same arithmetic as a 16-row call (AS moves with it in the staging below).  The
+     * A, as a 16-row call of this geometry would (AS moves with it in the staging below).  The
      * passes over a weight block are neighbours on one XCD (workgroups go round-robin over the
      * 8), so all but the first find it in the L2; the tail that 8 does not divide is in order. */
     const int passes = (M + 15) >> 4;

@@ -227,8 +227,10 @@ __device__ __forceinline__ bool prefill_f8_tile(const F8Args& P, uint8_t* smem, 
     uint8_t* const r0 = smem;
     uint8_t* const r1 = smem + L::STAGE;
     /* F8_CHAN: is every row's scale one finite value over the unit's groups?  Two lanes a row,
-     * each every other dword (the row may start inside one), 16 loads at once and ahead of the
-     * stages' so that their wait is not the stages' (one at a time cost 15 us a tile) */
+     * each every other dword, 16 loads at once and ahead of the stages' so that their wait is not
+     * the stages' (one at a time cost 15 us a tile).  A row may start or end inside a dword; its
+     * other half, at the plane's ends two bytes outside the operand, is read with it (an aligned
+     * dword lies in one page) and looked at by neither lane */
     uint32_t* const flag = reinterpret_cast<uint32_t*>(smem + L::LDS);
     constexpr int CB = 16;
     uint32_t cv[CB], c0 = 0;
