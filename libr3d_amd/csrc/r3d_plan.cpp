@@ -541,9 +541,19 @@ void prefill_geom(int64_t M, int64_t N, int64_t K, int mode, int ncu, PrefillGeo
     if (!narrow) {
         /* e2m1 weights on 128 x 128: a round costs 2.85 fragment-steps (0.54 us a step against
          * 0.87 of 128 x 256), so it runs where the larger tiles leave CUs idle (512 x 5376 x
-         * 5376: 168 tiles, 28 us, against 84 of 128 x 256, 41; at 714 tokens 30 against 42) */
-        const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128);
-        if ((double)((tiles + ncu - 1) / ncu) * 2.85 < best_cost) { best = 4; best_m = 2; }
+         * 5376: 168 tiles, 28 us, against 84 of 128 x 256, 41; at 714 tokens 30 against 42).
+         * Two and more of its rounds gain their shorter prologue over one and more of 192 x 256
+         * and lose at every step, where each larger tile's products share more operand bytes (us,
+         * 128 x 128 and 192 x 256; mxfp4a8 520 x 13056 x 1024 17.5 19.9, 315 x 20352 x 3840 50
+         * 53, 379 x 19456 x 5760 82 73, 1315 x 11008 x 8832, four rounds, 195 191; mxfp4a16
+         * 279 x 19584 x 1664 25.2 26.2, 381 x 20160 x 3328 46.9 44.8, 1098 x 6656 x 13696 173
+         * 143): up to 36 steps at two rounds, 20 at more, 18 at mxfp4a16. */
+        const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128), rounds = (tiles + ncu - 1) / ncu;
+        const int64_t most = mode == PF_MX8 ? 18 : rounds == 2 ? 36 : 20;
+        if ((double)rounds * 2.85 < best_cost && (rounds == 1 || K / 128 <= most)) {
+            best = 4;
+            best_m = 2;
+        }
     }
     g->wnf = best;
     g->wmf = best_m;

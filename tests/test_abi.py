@@ -736,6 +736,22 @@ def test_prefill_tile_choice_fills_the_last_round():
     assert g["bn"] == "128", g
 
 
+@pytest.mark.parametrize("dtype,M,N,K,bn,bm", [
+    # one round of 128 x 128 at any K; two up to 36 steps, more up to 20, at mxfp4a16 up to 18
+    ("mxfp4a8", 512, 7424, 21504, 128, 128), ("mxfp4a16", 512, 7424, 21504, 128, 128),
+    ("mxfp4a8", 379, 19456, 4608, 128, 128), ("mxfp4a8", 379, 19456, 4736, 192, 256),
+    ("mxfp4a8", 1825, 8448, 2560, 128, 128), ("mxfp4a8", 1825, 8448, 2688, 192, 256),
+    ("mxfp4a16", 1098, 6656, 2304, 128, 128), ("mxfp4a16", 1098, 6656, 2432, 192, 256),
+    ("mxfp4a16", 1282, 11136, 2304, 128, 128), ("mxfp4a16", 1282, 11136, 2432, 192, 256)])
+def test_e2m1_prefill_tile_by_rounds_and_steps(dtype, M, N, K, bn, bm):
+    if dtype == "mxfp4a16":
+        ops, keep, need = _a16_ops(M=M, N=N, K=K)
+    else:
+        ops, keep = _mx_ops(M=M, N=N, K=K)
+    g = _geom(R.describe("gemm_nt_q_mxfp4a16" if dtype == "mxfp4a16" else "gemm_nt_q_mxfp4", ops)[1])
+    assert (g["arm"], g["bn"], g["bm"]) == ("prefill", str(bn), str(bm)), g
+
+
 def test_a16_scratch_hook_and_refusals():
     ops, keep, need = _a16_ops()
     assert R.row_scratch_bytes("gemm_nt_q_mxfp4a16", ops) == need
