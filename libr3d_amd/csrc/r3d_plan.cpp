@@ -633,14 +633,27 @@ int prefill_f8_wide(int64_t M, int64_t N, int64_t K, int rblk, int ncu) {
     if (M <= 128 || f8_tile_lever()) return 0;
     if (ncu <= 0) ncu = 256;
     /* On the per-row grid the host cannot see whether the scales vary, so the wide tile runs
-     * where even its slower walk gains: M = 512, N = 21504, K = 5376 stays on the base tiles
-     * (109 us; the wide tile 93 with one scale a row, 128 with scales that vary). */
+     * where its slower walk gains too: M = 512, N = 21504, K = 5376 stays on the base tiles
+     * (109 us; the wide tile 93 with one scale a row, 128 with scales that vary).  Of 60 drawn
+     * launches of 256 x 256 two are slower where the scales vary (1483 x 8704 x 7808 166 -> 183,
+     * 1903 x 6784 x 11008 226 -> 233; with one scale a row 0.72 to 0.83 of the time on all). */
     const bool row = rblk == 1;
     const int64_t steps = K / 128;
     const int64_t base = f8_base_ns(row ? kF8BaseRow : kF8Base, M, N, steps, ncu);
     const int64_t c8 = f8_wide_ns(row ? kF8Wide8Row : kF8Wide8, 8, M, N, steps, 1, ncu);
-    const int64_t c4 = f8_wide_ns(row ? kF8Wide4Row : kF8Wide4, 4, M, N, steps, 1, ncu);
-    return c8 <= c4 ? (c8 < base ? 8 : 0) : c4 < base ? 4 : 0;
+    int64_t c4 = f8_wide_ns(row ? kF8Wide4Row : kF8Wide4, 4, M, N, steps, 1, ncu);
+    /* 256 x 128 against the four-wave 128 x 256 in no more rounds, the same products a round:
+     * scales that vary lose always (35 of 35, 2 to 13 %: 1370 x 3200 x 1536 23.2 -> 26.2 us,
+     * 150 x 20864 x 1152 18.9 -> 21.2; with one scale a row it gained 6 %); blocks gain up to 32
+     * steps (52 launches, 0.90 to 1.02 of the time) and past that as often lose (29, 0.93 to
+     * 1.13: 1136 x 4608 x 13824 123 -> 138). */
+    const int64_t r4 = f8_rounds(((N + 127) / 128) * ((M + 255) / 256), ncu);
+    if (r4 <= f8_rounds(((N + 255) / 256) * ((M + 127) / 128), ncu) && (row || steps > 32))
+        c4 = base;
+    /* two rounds of 256 x 256 for three of 128 x 256 are within the model's error (2016 x 10496 x
+     * 4992 on blocks 146 -> 154 us) */
+    if (c8 <= c4 && c8 * 100 < base * (row ? 100 : 90)) return 8;
+    return c4 < base ? 4 : 0;
 }
 
 PrefillGeom prefill_f8_geom(int wmw, int64_t M, int64_t N, int64_t K) {

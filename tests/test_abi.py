@@ -726,7 +726,7 @@ def test_prefill_tile_choice_fills_the_last_round():
     g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
     assert (g["waves"], g["nsplit"]) == ("4", "0"), g
     # where the planner runs the wide tile, the line is the wide tile's
-    for M, N, K, tile in [(512, 16640, 1024, ("256", "256", "8")), (512, 16384, 1024, ("256", "128", "8"))]:
+    for M, N, K, tile in [(512, 16640, 1024, ("256", "256", "8")), (300, 21504, 1024, ("256", "128", "8"))]:
         ops, _ = _f8_ops(M=M, N=N, K=K)
         g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
         assert (g["bn"], g["bm"], g["waves"], g["nsplit"]) == tile + ("0",), g
@@ -734,6 +734,20 @@ def test_prefill_tile_choice_fills_the_last_round():
     ops, _ = _mx_ops(M=256, N=4096, K=1024)
     g = _geom(R.describe("gemm_nt_q_mxfp4", ops)[1])
     assert g["bn"] == "128", g
+
+
+@pytest.mark.parametrize("rblk,M,N,K,wide", [
+    # 256 x 128 and the four-wave 128 x 256, one round of either: per row never, on blocks up to 32
+    # steps; where the former saves a round, at any K
+    (1, 1370, 3200, 1536, None), (128, 1370, 3200, 1536, "256x128"), (128, 1140, 4480, 4096, "256x128"),
+    (128, 1140, 4480, 4224, None), (128, 1136, 4608, 13824, None), (1, 339, 18688, 1792, "256x128"),
+    (128, 1353, 11520, 9088, "256x128"),
+    # 256 x 256: two rounds for three of 128 x 256 on blocks never, one for two on either grid
+    (128, 2016, 10496, 4992, None), (128, 1187, 8576, 1024, "256x256"), (1, 1187, 8576, 1024, "256x256")])
+def test_fp8_wide_tile_rule(rblk, M, N, K, wide):
+    ops, keep = _f8_ops(M=M, N=N, K=K, rblk=rblk)
+    g = _geom(R.describe("gemm_nt_q_fp8a8", ops)[1])
+    assert g["arm"] == "prefill" and g.get("wide") == wide, g
 
 
 @pytest.mark.parametrize("dtype,M,N,K,bn,bm", [
