@@ -16,8 +16,9 @@
  * The MFMA wants lane 16 kb + p to hold row p's chunks kb (lo) and 4 + kb (hi).  The two loads
  * take that form through 2 KB of the wave's own LDS (r3d_lines_turn).  Loading them in it
  * directly (each lane its own row, a select and two DPP rotates per register) takes the address
- * unit a row a lane: about 64 clocks a KB, which bounded a workgroup at 16 bytes a clock however
- * few of them ran (512 x 17152 at M = 14: 19.4 us e2m1 and 25.1 e4m3, 13.5 and 19.4 turned).
+ * unit a row a lane: about 64 clocks a KB (a bare loop, not kept), which bounded a workgroup at 16
+ * bytes a clock however few of them ran (512 x 17152 at M = 14: 19.4 us e2m1 and 25.1 e4m3, 13.5
+ * and 19.4 turned).
  *
  * For an fp8 operand (lo,
  * hi) are exactly the MFMA's bytes [16kb, +16) and [64 + 16kb, +16) of the lane's row;

@@ -27,9 +27,10 @@
  * Measured (us; before: 128 x 256 on four waves and 128 x 128, r3d_prefill.h):
  *   2048 x 21504 x 5376   128 x 128 blocks 283 -> 251, one scale a row 343 -> 258
  *                         (1.83 PFLOP/s), scales that vary along a row 353 -> 340
- *   512 x 5376 x 21504    (K split six ways, r3d_plan.cpp) 131 -> 86, 168 -> 89, 169 -> 129
+ *   512 x 5376 x 21504    (K split six ways, r3d_plan.cpp; with the planes' sum, 11 of it)
+ *                         133 -> 89, 168 -> 94, 169 -> 120
  * At full load the clock gives way before anything else: the same walk with no loads and no
- * LDS reads at all takes 1.83 us a step on 256 CUs and 1.15 on 42. */
+ * LDS reads at all (a variant, not kept) takes 1.83 us a step on 256 CUs and 1.15 on 42. */
 #ifndef R3D_PREFILL_F8_H
 #define R3D_PREFILL_F8_H
 
